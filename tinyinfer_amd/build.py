@@ -100,7 +100,7 @@ def build_oracle() -> None:
     """Compile oracle/ (the CPU checker) and, where the reference checkout exists,
     oracle/_ref (the reference's own CPU sources)."""
     _run(["make", "-s", "-C", str(ROOT / "oracle"), "all"])
-    if Path("/root/reference").is_dir():
+    if Path("/root/reference/kernels").is_dir():
         _run(["make", "-s", "-C", str(ROOT / "oracle"), "ref"])
 
 
