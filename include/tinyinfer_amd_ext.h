@@ -22,7 +22,7 @@ int ti_amd_gemm_i8_fused(const uint16_t* a, const int8_t* q, const float* scales
 /* ti_amd_legacy_gemm_f32_variant: the three FP32 GEMM variants behind
  * ikernels.cuda_bench_matmul(variant, ...) (reference
  * kernels/src/cuda/bench_api.cu:43-51 over kernels/src/cuda/matmul.cu:7-80):
- * 0 naive, 1 LDS-tiled, 2 register-tiled (what ti_cuda_gemm and
+ * 0 naive, 1 LDS-tiled, 2 MFMA-tiled (what ti_cuda_gemm and
  * ti_v2_legacy_gemm_f32 run).  y[M,N] = a[M,K] @ b[K,N] in fp32, device
  * pointers, v2 status codes (3 for an unknown variant). */
 int ti_amd_legacy_gemm_f32_variant(int variant, const float* a, const float* b, float* y, int m, int n, int k,

@@ -555,6 +555,26 @@ def test_legacy_fp32_gemm(ops):
         assert np.allclose(out, a.astype(np.float64) @ b, atol=1e-5 * k + 1e-5)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (512, 512, 127), (33, 31, 129), (16, 1000, 2048),       # 32 x 32 tiles, eight waves over K
+    (544, 520, 64), (700, 700, 1),                          # 32 x 32 tiles, four waves
+    (768, 768, 40), (1000, 1001, 33), (1089, 1024, 97),     # 64 x 64 tiles, with and without 16-byte rows
+    (1100, 1028, 68), (1600, 1284, 4),                      # 32 x 64 tiles
+    (2048, 2048, 31), (2049, 2050, 65),                     # 128 x 128 tiles
+])
+def test_legacy_fp32_gemm_tiles(ops, m, n, k):
+    """Each tile choice at ragged edges, against 64-bit sums.  A k-term fp32 sum
+    in any order is within k 2^-24 of sum |a b| (Higham, gamma_k)."""
+    t = torch()
+    say("fp32 gemm tiles", m, n, k)
+    gen = t.Generator(device="cuda").manual_seed(m + n + k)
+    a = t.randn(m, k, generator=gen, device="cuda")
+    b = t.randn(k, n, generator=gen, device="cuda")
+    out = ops.legacy_gemm(a, b).double()
+    bound = (k + 1) * 2.0 ** -24 * (a.abs().double() @ b.abs().double())
+    assert bool(((out - a.double() @ b.double()).abs() <= bound).all())
+
+
 # ---------------------------------------------------------------- attention
 @pytest.mark.parametrize("config", [0, 1])
 @pytest.mark.parametrize("d", [64, 128])

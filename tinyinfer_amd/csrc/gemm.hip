@@ -1987,47 +1987,183 @@ __global__ __launch_bounds__(256) void legacy_f32_tiled_kernel(const float* a, c
   if (row < m && col < n) c[row * n + col] = acc;
 }
 
-// Variant 2 (ti_cuda_gemm, ti_v2_legacy_gemm_f32): 64x64 output tile per
-// 256-thread block, 4x4 outputs per thread, K in 16-wide LDS slabs.
-__global__ __launch_bounds__(256) void legacy_f32_kernel(const float* a, const float* b, float* c,
-                                                         int m, int n, int k) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Bs[16][64 + 4];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int row0 = blockIdx.y * 64, col0 = blockIdx.x * 64;
-  float acc[4][4] = {};
-  for (int64_t k0 = 0; k0 < k; k0 += 16) {
+// Variant 2 (ti_cuda_gemm, ti_v2_legacy_gemm_f32): fp32 MFMA
+// (v_mfma_f32_16x16x4_f32: every product and sum in fp32).  A workgroup of
+// WM x WN x KG waves owns a BM x BN tile; K runs in slabs of BK through two LDS
+// buffers, the next two slabs in registers (their loads in flight during a
+// slab's MFMAs), one barrier per slab.  Lane (j, g) takes k = 4g .. 4g + 3 of a
+// 16-row step, so A is one ds_read_b128 per block and step, and MFMA i of the
+// step multiplies k = {i, 4 + i, 8 + i, 12 + i}.  B is read as four words of
+// row-major rows; the pitch BN + 4 (= 4 mod 16 words) puts the 64 lanes of each
+// read, and the pitch BK + 4 those of an A read, in 64 distinct banks.  KG > 1
+// (few tiles): the waves also share each slab's steps, and their sums meet in
+// LDS at the end, in wave order.  AV / BV: rows of A / B allow 16-byte loads.
+// Bound: the fp32 matrix rate (157 TF/s nominal, 135 by a large library product
+// here); what is lost goes to the barrier per slab (1024 MFMA cycles at 64 x 64).
+template <int BM, int BN, int WM, int WN, int KG, int BK, bool AV, bool BV>
+__global__ __launch_bounds__(WM * WN * KG * 64) void f32_mfma_kernel(const float* a, const float* b, float* c, int m,
+                                                                     int n, int k) {
+  constexpr int NT = WM * WN * KG * 64, MT = BM / WM / 16, RT = BN / WN / 16;
+  constexpr int PA = BK + 4, PB = BN + 4, STEPS = BK / 16;
+  constexpr int LA = BM * BK / 4 / NT, LB = BK * BN / 4 / NT;  // float4s per thread and slab
+  static_assert(LA >= 1 && LB >= 1 && BM * BK % (4 * NT) == 0 && BK * BN % (4 * NT) == 0, "whole float4s per thread");
+  static_assert(STEPS % KG == 0, "every K group takes the same steps");
+  constexpr int kStage = BM * PA + BK * PB;
+  static_assert(KG == 1 || (KG - 1) * BM * BN <= 2 * kStage, "the K groups' sums fit the buffers");
+  __shared__ __attribute__((aligned(16))) float lds[2 * kStage];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 15, g = lane >> 4;
+  const int kg = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  // Workgroups reach the 8 XCDs round-robin by linear id: each XCD gets one
+  // contiguous run of tiles, so its L2 holds the few A rows the run shares.
+  int tx, ty;
+  {
+    const int gx = int(gridDim.x), total = gx * int(gridDim.y), id = int(blockIdx.x) + gx * int(blockIdx.y);
+    const int n8 = total & ~7, li = id < n8 ? (id & 7) * (n8 >> 3) + (id >> 3) : id;
+    ty = li / gx;
+    tx = li - ty * gx;
+  }
+  const int row0 = ty * BM, col0 = tx * BN;
+
+  struct Slab {
+    float4_t a[LA], b[LB];
+  };
+  // Elements past M, N or K are zero in both operands.
+  auto load = [&](Slab& s, int64_t k0) {
 #pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      const int i = tid + l * 256;
-      const int ar = i >> 4, ak = i & 15;  // A tile 64 x 16
-      const int64_t gr = row0 + ar, gk = k0 + ak;
-      As[ak][ar] = (gr < m && gk < k) ? a[gr * k + gk] : 0.f;
-      const int bk = i >> 6, bc = i & 63;  // B tile 16 x 64
-      const int64_t gk2 = k0 + bk, gc = col0 + bc;
-      Bs[bk][bc] = (gk2 < k && gc < n) ? b[gk2 * n + gc] : 0.f;
+    for (int i = 0; i < LA; ++i) {
+      const int idx = tid + i * NT, r = row0 + idx / (BK / 4);
+      const int64_t kk = k0 + idx % (BK / 4) * 4;
+      const float* p = a + int64_t(r) * k + kk;
+      float4_t v = {0.f, 0.f, 0.f, 0.f};
+      if (r < m) {
+        if (AV) {
+          if (kk < k) v = *reinterpret_cast<const float4_t*>(p);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (kk + e < k) v[e] = p[e];
+        }
+      }
+      s.a[i] = v;
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const int idx = tid + i * NT, cc = col0 + idx % (BN / 4) * 4;
+      const int64_t kk = k0 + idx / (BN / 4);
+      const float* p = b + kk * n + cc;
+      float4_t v = {0.f, 0.f, 0.f, 0.f};
+      if (kk < k) {
+        if (BV) {
+          if (cc < n) v = *reinterpret_cast<const float4_t*>(p);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (cc + e < n) v[e] = p[e];
+        }
+      }
+      s.b[i] = v;
+    }
+  };
+  auto store = [&](const Slab& s, int buf) {
+    float* as = lds + buf * kStage;
+    float* bs = as + BM * PA;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const int idx = tid + i * NT;
+      *reinterpret_cast<float4_t*>(as + idx / (BK / 4) * PA + idx % (BK / 4) * 4) = s.a[i];
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const int idx = tid + i * NT;
+      *reinterpret_cast<float4_t*>(bs + idx / (BN / 4) * PB + idx % (BN / 4) * 4) = s.b[i];
+    }
+  };
+
+  float4_t acc[MT][RT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[t][r] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const int slabs = (k - 1) / BK + 1;
+  Slab s0, s1;
+  load(s0, 0);
+  store(s0, 0);
+  if (slabs > 1) load(s1, BK);
+  if (slabs > 2) load(s0, int64_t(2) * BK);
+  // Slab i from buffer i & 1, while slab i + 1 goes from its registers to the
+  // other buffer (free since the barrier) and slab i + 3 is requested into them.
+  auto step = [&](int i, Slab& next) {
+    __syncthreads();
+    const float* as = lds + (i & 1) * kStage + (wm * MT * 16 + j) * PA + 4 * g;
+    const float* bs = lds + (i & 1) * kStage + BM * PA + 4 * g * PB + wn * RT * 16 + j;
+    float4_t af[2][MT];
+    float bf[2][RT][4];
+    auto frags = [&](int q) {
+      const int k0 = (q * KG + kg) * 16;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) af[q & 1][t] = *reinterpret_cast<const float4_t*>(as + t * 16 * PA + k0);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bf[q & 1][r][e] = bs[(k0 + e) * PB + 16 * r];
+    };
+    frags(0);
+#pragma unroll
+    for (int q = 0; q < STEPS / KG; ++q) {
+      if (q + 1 < STEPS / KG) frags(q + 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[q & 1][t][e], bf[q & 1][r][e], acc[t][r], 0, 0, 0);
+      // (After the first step's fragment reads, which the MFMAs wait for.)
+      if (q == 0) {
+        if (i + 1 < slabs) store(next, (i + 1) & 1);
+        if (i + 3 < slabs) load(next, int64_t(i + 3) * BK);
+      }
+    }
+  };
+  for (int i = 0; i < slabs; i += 2) {
+    step(i, s1);
+    if (i + 1 < slabs) step(i + 1, s0);
+  }
+  if constexpr (KG > 1) {
+    __syncthreads();
+    auto at = [&](int grp, int t, int r, int v) {
+      return lds + (grp - 1) * BM * BN + (((wm * WN + wn) * MT + t) * RT + r) * 256 + v * 64 + lane;
+    };
+    if (kg > 0) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) *at(kg, t, r, v) = acc[t][r][v];
     }
     __syncthreads();
+    if (kg > 0) return;
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float av[4], bv[4];
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[kk][ty * 4 + i];
+      for (int r = 0; r < RT; ++r)
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) bv[jj] = Bs[kk][tx * 4 + jj];
+        for (int v = 0; v < 4; ++v)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) acc[i][jj] += av[i] * bv[jj];
-    }
-    __syncthreads();
+          for (int grp = 1; grp < KG; ++grp) acc[t][r][v] += *at(grp, t, r, v);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int64_t r = row0 + ty * 4 + i, cc = col0 + tx * 4 + jj;
-      if (r < m && cc < n) c[r * n + cc] = acc[i][jj];
+    for (int v = 0; v < 4; ++v) {
+      const int64_t row = row0 + (wm * MT + t) * 16 + 4 * g + v;
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const int col = col0 + (wn * RT + r) * 16 + j;
+        if (row < m && col < n) c[row * n + col] = acc[t][r][v];
+      }
     }
 }
 
@@ -2845,6 +2981,39 @@ hipError_t launch_tiled(const GemmArgs& g, bool wvec, bool avec, const Scratch* 
   return hipGetLastError();
 }
 
+template <int BM, int BN, int WM, int WN, int KG, int BK>
+void launch_f32_cfg(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t stream) {
+  const bool av = k % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0;
+  const bool bv = n % 4 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+  const dim3 grid(unsigned((n - 1) / BN + 1), unsigned((m - 1) / BM + 1)), block(WM * WN * KG * 64);
+  if (av && bv) hipLaunchKernelGGL((f32_mfma_kernel<BM, BN, WM, WN, KG, BK, true, true>), grid, block, 0, stream, a, b, c, m, n, k);
+  else if (av) hipLaunchKernelGGL((f32_mfma_kernel<BM, BN, WM, WN, KG, BK, true, false>), grid, block, 0, stream, a, b, c, m, n, k);
+  else if (bv) hipLaunchKernelGGL((f32_mfma_kernel<BM, BN, WM, WN, KG, BK, false, true>), grid, block, 0, stream, a, b, c, m, n, k);
+  else hipLaunchKernelGGL((f32_mfma_kernel<BM, BN, WM, WN, KG, BK, false, false>), grid, block, 0, stream, a, b, c, m, n, k);
+}
+
+// Tile by the number of workgroups it leaves (M x K x N, us; before: one
+// 64 x 64 tile of scalar fmas per workgroup for every shape):
+// * 128 x 128 from one full round of them: 2048^3 138 (124 TF/s; before 351);
+//   with too few, half the CUs idle (1024^3: 71);
+// * 32 x 32, eight waves sharing K, up to one round: 512 x 2048 x 512 20
+//   against 44 as 64 x 64 tiles (before 300), 300 x 1500 x 200 15 against 33;
+// * 32 x 32, four waves, while 64 x 64 tiles would fill less than half the CUs;
+// * 64 x 64 up to one round of them: 1024^3 25 (85 TF/s; before 163);
+// * 32 x 64, K over four waves, above that, where the last round of larger
+//   tiles would be thin: 2048 x 2048 x 640 64 against 78, 1536^3 80 against 87.
+//   Rows that allow no 16-byte loads keep 64 x 64 (1000 x 1003 x 1001: 35
+//   against 47): their loads cost more per tile.
+void launch_f32_mfma(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t stream) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); };
+  if (tiles(128, 128) >= 256) return launch_f32_cfg<128, 128, 2, 2, 2, 32>(a, b, c, m, n, k, stream);
+  if (tiles(32, 32) <= 256) return launch_f32_cfg<32, 32, 1, 1, 8, 128>(a, b, c, m, n, k, stream);
+  if (tiles(64, 64) < 128) return launch_f32_cfg<32, 32, 1, 1, 4, 64>(a, b, c, m, n, k, stream);
+  if (tiles(64, 64) > 256 && k % 4 == 0 && n % 4 == 0)
+    return launch_f32_cfg<32, 64, 1, 2, 4, 64>(a, b, c, m, n, k, stream);
+  return launch_f32_cfg<64, 64, 4, 2, 1, 32>(a, b, c, m, n, k, stream);
+}
+
 }  // namespace
 
 hipError_t gemm(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* deferred) {
@@ -2970,9 +3139,8 @@ hipError_t legacy_gemm_f32_variant(int variant, const float* a, const float* b, 
                                    hipStream_t stream) {
   if (m <= 0 || n <= 0 || k <= 0) return hipErrorInvalidValue;
   if (variant == 2) {
-    if ((m + 63) / 64 > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(legacy_f32_kernel, dim3(unsigned((n + 63) / 64), unsigned((m + 63) / 64)), dim3(256), 0,
-                       stream, a, b, c, m, n, k);
+    if ((m - 1) / 64 + 1 > 65535) return hipErrorInvalidValue;
+    launch_f32_mfma(a, b, c, m, n, k, stream);
   } else if (variant == 0 || variant == 1) {
     if ((m + 15) / 16 > 65535) return hipErrorInvalidValue;
     const dim3 grid(unsigned((n + 15) / 16), unsigned((m + 15) / 16));

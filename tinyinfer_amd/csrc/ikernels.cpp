@@ -171,7 +171,7 @@ PYBIND11_MODULE(ikernels, m) {
   m.def("cuda_device_available", &device_available);
   m.def("cuda_bench_matmul", &bench_matmul, py::arg("variant"), py::arg("M"), py::arg("N"), py::arg("K"),
         py::arg("iters") = 20,
-        "HIP-event ms per launch of FP32 GEMM variant 0 (naive), 1 (LDS-tiled) or 2 (register-tiled)");
+        "HIP-event ms per launch of FP32 GEMM variant 0 (naive), 1 (LDS-tiled) or 2 (MFMA-tiled)");
   m.def("cuda_bench_softmax", &bench_softmax, py::arg("rows"), py::arg("cols"), py::arg("iters") = 50);
   m.def("cuda_bench_layernorm", &bench_layernorm, py::arg("rows"), py::arg("cols"), py::arg("iters") = 50);
 }
