@@ -1007,3 +1007,30 @@ def test_non_default_stream_and_input_lifetime(ops):
     del tmp, tmp2, blocker
     default.wait_stream(stream)
     close(host(actual), expected)
+
+
+def test_attention_metadata_follows_the_stream(ops):
+    """Back-to-back calls with other lengths, none waited for: each call's
+    metadata reaches its own kernel (equal to the same call alone), and a call
+    under graph capture is refused before anything is queued."""
+    t = torch()
+    gen = t.Generator(device="cuda").manual_seed(3)
+    q, k, v = (t.randn(4, 2, n, 64, generator=gen, device="cuda").half() for n in (1, 96, 96))
+    cases = [[1 + (7 * i + 13 * b) % 96 for b in range(4)] for i in range(24)]
+    call = lambda lens: ops.attention(q, k, v, kv_lengths=lens, query_offsets=[n - 1 for n in lens])
+    alone = []
+    for lens in cases:
+        alone.append(call(lens))
+        t.cuda.synchronize()
+    side = t.cuda.Stream()
+    side.wait_stream(t.cuda.current_stream())
+    with t.cuda.stream(side):
+        queued = [call(lens) for lens in cases]
+    side.synchronize()
+    assert all(t.equal(a, b) for a, b in zip(alone, queued))
+    with t.cuda.stream(side):
+        graph = t.cuda.CUDAGraph()
+        with pytest.raises(RuntimeError, match="captured"):
+            with t.cuda.graph(graph, stream=side):
+                call(cases[0])
+    assert t.equal(call(cases[1]), alone[1])
