@@ -24,6 +24,7 @@ import itertools
 import json
 import math
 from array import array
+from contextlib import nullcontext
 from pathlib import Path
 
 from . import BACKEND_LIB, require
@@ -160,7 +161,9 @@ class _Call:
         memory would wait for everything queued on the stream before it; three
         such copies made a 32-request decode call 73 us, this one 27)."""
         torch = self.ops.torch
-        if torch.cuda.is_current_stream_capturing():
+        with torch.cuda.device(self.device) if torch.cuda.current_device() != self.device.index else nullcontext():
+            capturing = torch.cuda.is_current_stream_capturing()
+        if capturing:
             raise RuntimeError(f"{self.symbol}: host metadata cannot be captured into a graph")
         flat = array("i", itertools.chain(*lists))
         host = torch.empty(len(flat), dtype=torch.int32, pin_memory=True)
