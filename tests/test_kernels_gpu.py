@@ -544,6 +544,94 @@ def test_layernorm_prologue_gemv_rejects_unsupported_shapes(ops):
     assert _ln_packed(*args(0, 64)) == 1
 
 
+# m, n, k of each tile choice of the large products, at ragged edges: 64-row tiles
+# (int8 over and up to 1024 rows, fp16), 128 x 128, 128 x 256 (int8), 256 x 256
+# in one round, and 256 x 256 tiles whose last round is 128-row tiles.
+LARGE = [(1030, 260, 200), (1000, 1300, 136), (640, 644, 264), (1100, 2052, 72), (2047, 2560, 40),
+         (3601, 3844, 72), (5000, 3844, 40)]
+
+
+def large_reference(a, w, bias):
+    """64-bit product, and the bound on an fp32 sum of its terms in any order
+    (k + 2 roundings of at most 2^-24 of sum |a w| + |bias|)."""
+    ref = a.double() @ w.double() + bias.double()
+    size = a.abs().double() @ w.abs().double() + bias.abs().double()
+    return ref, (a.shape[1] + 2) * 2.0 ** -24 * size
+
+
+def large_operands(m, n, k, seed):
+    t = torch()
+    gen = t.Generator(device="cuda").manual_seed(seed)
+    a = t.randn(m, k, generator=gen, device="cuda").half()
+    q = t.randint(-127, 128, (k, n), generator=gen, device="cuda", dtype=t.int8)
+    s = t.rand(n, generator=gen, device="cuda") * 1e-3 + 1e-3
+    bias = t.randn(n, generator=gen, device="cuda").half()
+    return a, q, s, (q.float() * s).half(), bias
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("m,n,k", LARGE)
+def test_row_major_large_tiles(ops, m, n, k, int8):
+    """fp32 and fp16 outputs, fused and separate bias, and a row that holds an
+    infinity: it must not leak through the K padding or into other rows."""
+    t = torch()
+    say("row-major large tiles", m, n, k, int8)
+    a, q, s, w, bias = large_operands(m, n, k, m + n + k)
+    ref, bound = large_reference(a, w, bias)
+    call = lambda x, **kw: ops.gemm_int8(x, q, s, **kw) if int8 else ops.gemm(x, w, **kw)
+    out = call(a, bias=bias, output_dtype=t.float32)
+    assert bool(((out.double() - ref).abs() <= bound).all())
+    assert t.equal(call(a, bias=bias, config=6, output_dtype=t.float32), out)
+    assert t.equal(call(a, bias=bias), out.half())
+    bad = a.clone()
+    bad[m - 2, k - 1] = float("inf")
+    got = call(bad, output_dtype=t.float32)
+    keep = t.arange(m, device="cuda") != m - 2
+    assert t.equal(got[keep], call(a, output_dtype=t.float32)[keep])
+    want = t.where(w[k - 1] == 0, float("nan"), t.sign(w[k - 1].float()) * float("inf"))
+    assert t.equal(got[m - 2].nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("m,n,k", LARGE)
+def test_row_major_large_tiles_fused(ops, m, n, k):
+    """GELU and residual epilogues, aligned outputs and ones that allow no wide
+    store, against the plain output's own 16-bit values."""
+    t = torch()
+    say("row-major large tiles fused", m, n, k)
+    a, q, s, w, bias = large_operands(m, n, k, m + n + k)
+    plain = ops.gemm_int8(a, q, s, bias=bias)
+    res = t.randn(m, n, device="cuda").half()
+    for off in (0, 1):
+        y = t.empty(m * n + 8, dtype=t.float16, device="cuda")[off:off + m * n].view(m, n)
+        _fused(ops.lib, a, q, s, bias, y, res, m, n, k, 2)
+        assert t.equal(y, (res.float() + plain.float()).half())
+        _fused(ops.lib, a, q, s, bias, y, None, m, n, k, 1)
+        z = plain.double()
+        gelu = 0.5 * z * (1 + t.tanh(0.7978845608028654 * (z + 0.044715 * z ** 3)))
+        # 2e-7 absolute on the tanh, half an fp16 step on the result.
+        assert bool(((y.double() - gelu).abs() <= 2.0 ** -11 * gelu.abs() + 1e-6 * z.abs() + 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1100, 2050, 96), (3601, 3841, 160), (5000, 3844, 32), (1100, 2050, 64)])
+def test_record_large_tiles(ops, m, n, k):
+    """fp16 records: the value of every tile choice, and the bits of the
+    row-major kernel where that takes the shape (one K order everywhere)."""
+    t = torch()
+    say("record large tiles", m, n, k)
+    a, q, s, w, bias = large_operands(m, n, k, m + n + k)
+    packed = _pack16_gpu(ops.lib, q, s, k, n)
+    y = t.empty(m, n, dtype=t.float16, device="cuda")
+    assert _w16(ops.lib, a, packed, bias, y, None, m, n, k, 0) == 0
+    ref, bound = large_reference(a, w, bias)
+    assert bool(((y.double() - ref).abs() <= bound + 2.0 ** -11 * (ref.abs() + bound) + 2.0 ** -25).all())
+    if n % 4 == 0:
+        assert t.equal(y, ops.gemm_int8(a, q, s, bias=bias))
+    few = 600  # 64 x 64 tiles, unsplit
+    z = t.empty(few, n, dtype=t.float16, device="cuda")
+    assert _w16(ops.lib, a[:few].contiguous(), packed, bias, z, None, few, n, k, 0) == 0
+    assert t.equal(z, y[:few])
+
+
 def test_legacy_fp32_gemm(ops):
     t = torch()
     rng = np.random.default_rng(4)

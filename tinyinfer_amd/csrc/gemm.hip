@@ -31,7 +31,10 @@
 //    of the tile in the same launch (partials in the queue's slot of a static
 //    pool, written and read with agent-scope accesses, so no L2-wide
 //    writeback or invalidate is needed; queue_scratch.hpp).
-//  * tiled (M > 32 where the row GEMM does not apply, M > 1024): 64x64x32 tiles, A and the dequantised weight tile
+//  * large tiles (tile_gemm_kernel: row-major weights of either type and fp16
+//    records, where the grid of 64- to 256-row tiles fills the chip).
+//  * tiled (M > 32 where neither applies: unaligned operands, fp16 weights over
+//    few tiles): 64x64x32 tiles, A and the dequantised weight tile
 //    staged in LDS (weights transposed to [n][k] so both MFMA operands are one
 //    ds_read_b128 per lane), double buffered, same fused epilogues.
 // Dequantisation mirrors reference kernels/src/cuda/tc/gemm.cu:21,24 and the
@@ -2877,48 +2880,482 @@ hipError_t launch_f16_cfg(const GemmArgs& g, const Scratch* s, hipStream_t strea
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// Large-tile MFMA GEMM
+// ---------------------------------------------------------------------------
+// Weights of tile_gemm_kernel: fp16 B records (pack_w16), or the ABI's
+// row-major [K][N] in fp16 or int8.
+enum TileWeights : int { TW_REC16 = 0, TW_ROW16 = 1, TW_ROW8 = 2 };
+
+// Zeros read in place of operand bytes past K.
+__device__ __attribute__((aligned(16))) const uint8_t kZero16[16] = {};
+
+struct TileParams {
+  const uint16_t* a;
+  int64_t lda;
+  const void* w;
+  const float* scales;
+  int m, n, k;
+  int64_t ldw;
+  int m_begin;               // first row of this launch's tiles
+  int tiles_n, tiles;
+  Epilogue epi;
+};
+// Tile rows per group of the tile order: the 32 tiles an XCD runs together
+// (256 x 256, one per CU) are 8 x 4, so its L2 fetches 12 operand panels a
+// chunk.  M = 8192, 1600->6400, int8: 207 us; groups of 2 / 4: 235 / 213.
+constexpr int kTileGroup = 8;
+
+// Tile (WM * MT * 16) x (WN * R * 16), WM x WN waves of MT x R MFMA blocks,
+// every output summed over K in 32-row MFMA steps from 0 upward whatever the
+// tile (so tile choices agree bit for bit).  What bounds it is keeping the
+// matrix cores fed: a 256 x 256 tile needs 1024 MFMA cycles per CU and 32 K
+// rows, against 96 KiB of LDS reads and 32 KiB of loads.
+//  * K runs in chunks of 64, one barrier per chunk.  A's loads go straight to
+//    LDS with 8 lanes on the 128 contiguous bytes of a row: a load of 16 rows x
+//    64 bytes in fragment order makes each 16-lane step of it touch 16 cache
+//    lines (M = 2560, 6400->1600: 122 us in that form, 80 in this one).  The
+//    16-byte pieces are exchanged as they land so that the fragment reads are
+//    free of bank conflicts.
+//  * Fragments are read a quarter chunk ahead of their MFMAs, the first of the
+//    next chunk right after the barrier, while the last quarter's MFMAs run.
+//  * fp16 records are already fragments and take the same direct loads.
+//    Row-major weights go through registers: a thread loads 4 columns of 8 K
+//    rows (a wave: 256 or 512 contiguous bytes per row), converts (int8:
+//    fp16_rn(float(q) * scale), 80 VALU per thread and chunk) and stores the
+//    four 8-row columns as fragments, between the MFMAs of the chunk's last two
+//    quarters.  Its 4 adjacent columns go to the same lane of 4 adjacent column
+//    blocks, which makes all loads and stores wide and conflict-free, and lane
+//    j's outputs 4 adjacent columns, stored without a pass through LDS.
+// M = 8192, 1600->6400: int8 row-major 517 -> 181 us (930 TF/s; the 64 x 64
+// kernel converted every weight once per 64 rows), fp16 row-major 511 -> 165 us,
+// fp16 records 228 -> 190 us; M = 2048, 768->3072, fp16 row-major 38 -> 19 us.
+template <int TW, int WM, int WN, int MT, int R, int EP, int OCC>
+__global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams p) {
+  constexpr int W = WM * WN, NT = W * 64;
+  constexpr int BM = WM * MT * 16, BN = WN * R * 16, H = MT / 2;
+  constexpr bool REC = TW == TW_REC16, Q8 = TW == TW_ROW8;
+  constexpr int SB = REC ? 2 : 3;                   // stages of W (A: 2)
+  constexpr int ASTAGE = BM * 128, BSTAGE = BN * 128;
+  constexpr int LA = BM / 8 / W, LB = BN / 8 / W;   // KiB loads per wave and chunk
+  constexpr int UN = BN * 2 / NT;                   // row-major W: 8 x 4 units per thread and chunk
+  static_assert(BM % (8 * W) == 0 && MT % 2 == 0, "whole A loads per wave, two halves of A blocks");
+  static_assert(REC ? BN % (8 * W) == 0 : (UN >= 1 && BN * 2 % NT == 0 && R == 4), "W loads split evenly");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // 2 A stages, SB W stages
+  uint8_t* const blds = lds + 2 * ASTAGE;
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  // Each XCD (workgroups go to them round-robin) takes one contiguous run of
+  // tiles, walked in groups of kTileGroup tile rows, column by column.
+  int tm, tn;
+  {
+    const int nbk = int(gridDim.x), bid = int(blockIdx.x), q = nbk >> 3, rem = nbk & 7, x = bid & 7;
+    const int tile = x * q + min(x, rem) + (bid >> 3);
+    const int tiles_m = p.tiles / p.tiles_n;
+    const int per_group = kTileGroup * p.tiles_n, group = tile / per_group, first = group * kTileGroup;
+    const int gm = min(tiles_m - first, kTileGroup), r = tile - group * per_group;
+    tm = first + r % gm;
+    tn = r / gm;
+  }
+  const int m0 = p.m_begin + tm * BM, n0 = tn * BN;
+  const int kc = (p.k + 63) / 64, kh = (p.k + 31) / 32;  // chunks, 32-row record groups
+
+  // A load covers 8 rows x 64 K.  LDS row 2 (r & 7) + (r >> 3) of a 16-row
+  // block holds block row r, its 16-byte piece s at s ^ (r & 7): the 16 lanes of
+  // a fragment read (16 rows, one piece) fall on 16 different 16-byte columns.
+  const char* const abase = reinterpret_cast<const char*>(p.a + int64_t(m0) * p.lda);
+  uint32_t aoff[LA];
+  auto load_row = [&](int l) {  // block row of this lane's part of load l
+    const int at = ((wave * LA + l) & 1) * 8 + (lane >> 3);
+    return (at >> 1) + 8 * (at & 1);
+  };
+#pragma unroll
+  for (int l = 0; l < LA; ++l) {
+    const int r = load_row(l);
+    aoff[l] = uint32_t(min((wave * LA + l) / 2 * 16 + r, p.m - 1 - m0)) * uint32_t(p.lda) * 2u +
+              16u * ((lane & 7) ^ (r & 7));
+  }
+  auto issue_a = [&](int c) {
+    uint8_t* st = lds + (c & 1) * ASTAGE + wave * LA * 1024;
+    const char* base = abase + int64_t(c) * 128;
+    if (c * 64 + 64 <= p.k) {
+#pragma unroll
+      for (int l = 0; l < LA; ++l)
+        __builtin_amdgcn_global_load_lds((global_ptr)(base + aoff[l]), (lds_ptr)(st + l * 1024), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int l = 0; l < LA; ++l) {
+        const char* s = base + aoff[l];
+        if (c * 64 + 8 * ((lane & 7) ^ (load_row(l) & 7)) >= p.k) s = reinterpret_cast<const char*>(kZero16);
+        __builtin_amdgcn_global_load_lds((global_ptr)s, (lds_ptr)(st + l * 1024), 16, 0, 0);
+      }
+    }
+  };
+  // W records: load id = 2 cb + s is K group s of the chunk of column block cb.
+  const char* wsrc[REC ? LB : 1];
+  if constexpr (REC) {
+    const int nbt = (p.n + 15) / 16;
+#pragma unroll
+    for (int l = 0; l < LB; ++l)
+      wsrc[l] = static_cast<const char*>(p.w) + int64_t(min(n0 / 16 + (wave * LB + l) / 2, nbt - 1)) * kh * 1024 + lane * 16;
+  }
+  auto issue_w = [&](int c) {
+#pragma unroll
+    for (int l = 0; l < (REC ? LB : 0); ++l) {
+      const int id = wave * LB + l, group = 2 * c + (id & 1);
+      const char* s = group < kh ? wsrc[l] + int64_t(group) * 1024 : reinterpret_cast<const char*>(kZero16);
+      __builtin_amdgcn_global_load_lds((global_ptr)s, (lds_ptr)(blds + (c & 1) * BSTAGE + id * 1024), 16, 0, 0);
+    }
+  };
+  // Row-major W unit u of a thread: columns col .. col + 3 (clamped into the
+  // row) of K rows 8 uoct .. + 7 of a chunk.
+  constexpr int UPR = BN / 4, WB = Q8 ? 1 : 2;
+  typedef uint32_t WRow __attribute__((ext_vector_type(Q8 ? 1 : 2)));
+  struct Raw {
+    WRow r[REC ? 1 : UN][8];
+  };
+  uint32_t uoff[REC ? 1 : UN];
+  int uoct[REC ? 1 : UN];
+  float usc[REC ? 1 : UN][4];
+  uint8_t* udst[REC ? 1 : UN];
+  if constexpr (!REC) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int id = int(threadIdx.x) + u * NT, cu = id % UPR, col = min(n0 + 4 * cu, (p.n + 3) / 4 * 4 - 4);
+      uoct[u] = id / UPR;
+      uoff[u] = (uint32_t(8 * uoct[u]) * uint32_t(p.ldw) + uint32_t(col)) * WB;
+      udst[u] = blds + ((cu >> 4) * 8 + (uoct[u] >> 2)) * 1024 + ((cu & 15) + 16 * (uoct[u] & 3)) * 16;
+      if constexpr (Q8) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) usc[u][c] = p.scales[min(col + c, p.n - 1)];
+      }
+    }
+  }
+  auto load_w = [&](Raw& raw, int c) {
+    if constexpr (!REC) {
+      const char* base = static_cast<const char*>(p.w) + int64_t(c) * 64 * p.ldw * WB;
+      if (c * 64 + 64 <= p.k) {
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            raw.r[u][e] = *reinterpret_cast<const WRow*>(base + int64_t(e) * p.ldw * WB + uoff[u]);
+      } else {
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            raw.r[u][e] = WRow(0);
+            if (c * 64 + 8 * uoct[u] + e < p.k)
+              raw.r[u][e] = *reinterpret_cast<const WRow*>(base + int64_t(e) * p.ldw * WB + uoff[u]);
+          }
+      }
+    }
+  };
+  // Column cc of every unit, as the 8 K rows of its lane of a B fragment.
+  auto store_col = [&](const Raw& raw, int stage, int cc) {
+    if constexpr (!REC) {
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (Q8) {
+            const uint32_t word = raw.r[u][e][0];
+            float x = float(int32_t(word << (24 - 8 * cc)) >> 24) * usc[u][cc];
+            asm("" : "+v"(x));  // rounded to fp32 first, as f16r
+            o[e] = f16(x);
+          } else {
+            o[e] = __builtin_bit_cast(f16, uint16_t(raw.r[u][e][cc >> 1] >> (16 * (cc & 1))));
+          }
+        }
+        *reinterpret_cast<half8_t*>(udst[u] + stage * BSTAGE + cc * 2048) = o;
+      }
+    }
+  };
+
+  float4_t acc[MT][R];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[t][r] = float4_t{0.f, 0.f, 0.f, 0.f};
+  half8_t a0[H], a1[H], b0[R], b1[R];
+  const int afrag = (2 * (j & 7) + (j >> 3)) * 128 + ((g ^ (j & 7)) * 16);
+  // A blocks half H .. of the wave in 32-row half s of chunk c; its B blocks.
+  auto read_a = [&](half8_t (&f)[H], int c, int s, int half) {
+    const uint8_t* at = lds + (c & 1) * ASTAGE + (wm * MT + half * H) * 2048 + (afrag ^ (s * 64));
+#pragma unroll
+    for (int t = 0; t < H; ++t) f[t] = *reinterpret_cast<const half8_t*>(at + t * 2048);
+  };
+  auto read_b = [&](half8_t (&f)[R], int stage, int s) {
+    const uint8_t* at = blds + stage * BSTAGE + wn * R * 2048 + s * 1024 + lane * 16;
+#pragma unroll
+    for (int r = 0; r < R; ++r) f[r] = *reinterpret_cast<const half8_t*>(at + r * 2048);
+  };
+  Raw raw;
+  // One quarter chunk of MFMAs; `cols` >= 0: columns cols, cols + 1 of the
+  // units in `raw` are converted and stored between them.
+  auto quarter = [&](const half8_t (&fa)[H], const half8_t (&fb)[R], int half, int stage, int cols) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < H; ++t)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        acc[half * H + t][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa[t], fb[r], acc[half * H + t][r], 0, 0, 0);
+    if (!REC && cols >= 0) {
+      store_col(raw, stage, cols);
+      store_col(raw, stage, cols + 1);
+#pragma unroll
+      for (int i = 0; i < H * R; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                             // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, ((Q8 ? 40 : 8) * UN + H * R - 1) / (H * R), 0);  // VALU
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Every load and LDS access of this wave done, then the workgroup meets.
+  auto meet = [&]() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (c < kc) {
+      issue_a(c);
+      issue_w(c);
+      if constexpr (!REC) {
+        load_w(raw, c);
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) store_col(raw, c, cc);
+      }
+    }
+  meet();
+  int st0 = 0, st1 = 1, st2 = SB - 1;  // W stages of chunks c, c + 1 and (row-major) c + 2
+  read_b(b0, 0, 0);
+  read_a(a0, 0, 0, 0);
+  for (int c = 0; c < kc; ++c) {
+    if (!REC && c + 2 < kc) load_w(raw, c + 2);
+    read_a(a1, c, 0, 1);
+    quarter(a0, b0, 0, 0, -1);
+    read_b(b1, st0, 1);
+    read_a(a0, c, 1, 0);
+    quarter(a1, b0, 1, 0, -1);
+    read_a(a1, c, 1, 1);
+    // Stage st2 was chunk c - 1's: free since the last barrier.  (Past the last
+    // chunk stale values go there and are not read.)
+    quarter(a0, b1, 0, st2, 0);
+    // Chunk c + 1 has landed, and every wave holds all of chunk c.  (After the
+    // last chunk the fragments read here are stale and not used.)
+    meet();
+    if (c + 2 < kc) {
+      issue_a(c + 2);
+      issue_w(c + 2);
+    }
+    read_b(b0, st1, 0);
+    read_a(a0, c + 1, 0, 0);
+    quarter(a1, b1, 1, st2, 2);
+    if constexpr (REC) {
+      st0 ^= 1;
+      st1 ^= 1;
+    } else {
+      const int t = st0;
+      st0 = st1;
+      st1 = st2;
+      st2 = t;
+    }
+  }
+
+  if constexpr (REC) {
+    // Through an LDS fp32 tile of BM / EP rows x BN, EP passes.
+    float bias[4];
+    load_bias4(p.epi, n0 + 4 * int(threadIdx.x % (BN / 4)), p.n, p.a, bias);
+    constexpr int PR = BM / EP;
+    static_assert(BM % EP == 0 && PR % 16 == 0, "whole 16-row blocks per pass");
+    float* ctile = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int pass = 0; pass < EP; ++pass) {
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int rb = (wm * MT + t) * 16 - pass * PR;  // block row inside this pass
+        if (rb < 0 || rb >= PR) continue;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            ctile[(rb + 4 * g + v) * tile_pitch(BN) + (wn * R + r) * 16 + j] = acc[t][r][v];
+      }
+      __syncthreads();
+      tile_epilogue<PR, BN, NT>(p.epi, ctile, m0 + pass * PR, n0, p.m, p.n, bias, nullptr, 0);
+    }
+  } else {
+    // Lane (j, g): rows 4g + v of each block, columns 4j .. 4j + 3 of the wave's 64.
+    const int col = n0 + wn * 64 + 4 * j;
+    if (col >= p.n) return;
+    const Epilogue& e = p.epi;
+    float bias[4];
+    load_bias4(e, col, p.n, p.a, bias);
+    const bool full = col + 4 <= p.n;
+    with_epilogue_kind(e, [&](auto kind) {
+      constexpr int K = decltype(kind)::value;
+      constexpr bool F32 = K == EPI_RAW_F32 || K == EPI_F32;
+      if constexpr (K == EPI_QKV) return;  // (the dispatch keeps it on the other kernels)
+      const bool vec = full && e.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(e.y) % (F32 ? 16 : 8) == 0 &&
+                       (K != EPI_RESIDUAL || (e.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(e.residual) % 8 == 0));
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = m0 + (wm * MT + t) * 16 + 4 * g + v;
+          if (row >= p.m) continue;
+          if (!vec) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              if (col + c < p.n)
+                epilogue_k<K>(e, row, col + c, acc[t][c][v], bias[c],
+                              K == EPI_RESIDUAL ? h2f(e.residual[r_off(e, row, col + c)]) : 0.f);
+            continue;
+          }
+          if constexpr (F32) {
+            *reinterpret_cast<float4_t*>(static_cast<float*>(e.y) + int64_t(row) * e.ldy + col) =
+                float4_t{acc[t][0][v] + bias[0], acc[t][1][v] + bias[1], acc[t][2][v] + bias[2], acc[t][3][v] + bias[3]};
+          } else {
+            half4_t rs = {};
+            if constexpr (K == EPI_RESIDUAL) rs = *reinterpret_cast<const half4_t*>(e.residual + int64_t(row) * e.ldr + col);
+            half4_t o;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const float x = acc[t][c][v] + bias[c];
+              o[c] = f16r(K == EPI_GELU ? gelu_tanh(rt16(x)) : K == EPI_RESIDUAL ? float(rs[c]) + rt16(x) : x);
+            }
+            *reinterpret_cast<half4_t*>(static_cast<uint16_t*>(e.y) + int64_t(row) * e.ldy + col) = o;
+          }
+        }
+    });
+  }
+}
+
+// Rows [m_begin, m_end) of the product.
+template <int TW, int WM, int WN, int MT, int R, int EP, int OCC>
+hipError_t launch_tile_cfg(const GemmArgs& g, int m_begin, int m_end, hipStream_t stream) {
+  constexpr int BM = WM * MT * 16, BN = WN * R * 16;
+  constexpr bool REC = TW == TW_REC16;
+  constexpr size_t kRing = size_t(2) * BM * 128 + size_t(REC ? 2 : 3) * BN * 128;
+  constexpr size_t kLds = std::max(kRing, REC ? size_t(BM / EP) * tile_pitch(BN) * 4 : size_t(0));
+  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
+  if (attr != hipSuccess) return attr;
+  TileParams p{};
+  p.a = g.a; p.lda = g.lda; p.w = REC ? g.w_f16p : g.w; p.scales = g.scales;
+  p.m = m_end; p.n = g.n; p.k = g.k; p.epi = g.epi;
+  p.ldw = g.ldw > 0 ? g.ldw : g.n;
+  p.m_begin = m_begin;
+  p.tiles_n = (g.n + BN - 1) / BN;
+  const int64_t tiles = int64_t(p.tiles_n) * ((m_end - m_begin + BM - 1) / BM);
+  if (tiles > (int64_t(1) << 28)) return hipErrorInvalidValue;
+  p.tiles = int(tiles);
+  hipLaunchKernelGGL((tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>), dim3(unsigned(tiles)), dim3(WM * WN * 64), kLds,
+                     stream, p);
+  return hipGetLastError();
+}
+
+// Which tiles a large product takes: rows [0, big) as 256 x 256 tiles and the
+// rest as 128-row ones, `big` from a cost in rounds of 256 x 256 tiles over the
+// CUs.  128 x 128 tiles run two workgroups per CU at about 1.15 of the time per
+// output, plus about a third of a round to start and drain (MI355X, us):
+// * one full round: M = 8192, 6400->1600 (224 big tiles) 177 against 228 as
+//   128-row tiles; half a round or less: M = 2560, 6400->1600 148 against 80;
+// * a thin last round is replaced by 128-row tiles: M = 8192, 1600->6400 (800
+//   big tiles, 3.1 rounds) 181 against 207.
+int tile_big_rows(int m, int n) {
+  const int64_t cus = device_cus(), ct = (int64_t(n) + 255) / 256, rows = (int64_t(m) + 255) / 256;
+  auto mid = [&](int64_t from) {
+    if (from >= m) return 0.0;
+    return 0.35 + 1.15 / 4 * double((m - from + 127) / 128 * ((int64_t(n) + 127) / 128)) / double(cus);
+  };
+  auto big = [&](int64_t r) { return double((r * ct + cus - 1) / cus); };
+  int64_t best = 0;
+  double cost = mid(0);
+  if (big(rows) < cost) {
+    best = m;
+    cost = big(rows);
+  }
+  const int64_t full = rows * ct / cus * cus / ct;  // tile rows in whole rounds
+  if (full > 0 && full < rows && big(full) + mid(full * 256) < cost) best = full * 256;
+  return int(best);
+}
+int64_t tiles_of(int m, int n, int bm, int bn) {
+  return (int64_t(m) + bm - 1) / bm * ((int64_t(n) + bn - 1) / bn);
+}
+
+// The 128-row tiles: 128 x 256 where their grid makes one round at least 0.6
+// full (int8: the conversions are shared by twice the columns per barrier;
+// M = 2048, 768->3072 19.7 against 21.2 us as 128 x 128), else 128 x 128, two
+// workgroups per CU.
+template <int TW>
+hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
+  const int big = tile_big_rows(g.m, g.n);
+  if (big > 0) {
+    const hipError_t e = launch_tile_cfg<TW, 2, 4, 8, 4, 8, 2>(g, 0, std::min(big, g.m), stream);
+    if (e != hipSuccess || big >= g.m) return e;
+  }
+  if constexpr (TW == TW_REC16) {
+    return launch_tile_cfg<TW, 2, 4, 4, 2, 4, 4>(g, big, g.m, stream);
+  } else {
+    const int64_t wide = tiles_of(g.m - big, g.n, 128, 256), cus = device_cus();
+    if (TW == TW_ROW8 && 5 * wide >= 3 * cus && wide <= cus)
+      return launch_tile_cfg<TW, 2, 4, 4, 4, 4, 2>(g, big, g.m, stream);
+    return launch_tile_cfg<TW, 2, 2, 4, 4, 4, 2>(g, big, g.m, stream);
+  }
+}
+
+// Row-major weights over the large tiles, for operands that allow their wide
+// loads.  hipErrorNotSupported: the shape is better served by the kernels that
+// split K over few tiles (us, this kernel against them):
+// * int8 up to kRowMaxM rows (the row GEMM): from 160 tiles of 64 x 128:
+//   512 x 768 x 3072 12.4 / 14.9, 1024 x 1600 x 1600 21.5 / 25.2, 1024 x 768 x
+//   3072 15.1 / 25.8; below, 1024 x 768 x 768 12.1 / 9.8, 512 x 3072 x 768
+//   36 / 14.8; the longest K keeps the row GEMM up to 160 tiles of 128 x 128
+//   (1024 x 6400 x 1600 87 / 83);
+// * fp16 (the tiled kernel): from 100 tiles of 64 x 64: 256 x 768 x 3072 9.9 /
+//   14.2, 1024 x 3072 x 768 37 / 62; below, 128 x 768 x 768 9.6 / 8.7.
+template <int TW>
+hipError_t launch_row_tiles(const GemmArgs& g, hipStream_t stream) {
+  const int64_t ldw = g.ldw > 0 ? g.ldw : g.n;
+  if (g.k % 8 != 0 || g.lda > (1 << 22) || ldw > (1 << 24) || g.epi.kind == EPI_QKV || g.epi.p32 || g.m <= 32)
+    return hipErrorNotSupported;
+  const int64_t mid = tiles_of(g.m, g.n, 128, 128);
+  if (mid >= 144) return launch_tile<TW>(g, stream);
+  if constexpr (TW == TW_ROW8) {
+    if (g.m <= kRowMaxM && (tiles_of(g.m, g.n, 64, 128) < 160 || g.k > 4096)) return hipErrorNotSupported;
+    return launch_tile_cfg<TW, 2, 2, 2, 4, 2, 2>(g, 0, g.m, stream);
+  } else {
+    if (tiles_of(g.m, g.n, 64, 64) < 100) return hipErrorNotSupported;
+    return launch_tile_cfg<TW, 2, 1, 2, 4, 2, 2>(g, 0, g.m, stream);
+  }
+}
+
 // Tile choice over the fp16 records, and when they beat the int8 panel
 // kernel, from timings on MI355X (graph replays over rotating weights):
-// * 128 x 128 tiles on 8 waves (each 64 x 32, 3 stages, the epilogue in 4
-//   passes of 32 rows so three workgroups fit a CU) once the grid holds >= 384
-//   of them, or >= 192 at K >= 1536: M = 8192 1600->6400 247 us (679 TF/s;
-//   4 waves of 64 x 64: 309 us), 768->2304 65 us (64 x 64 tiles: 76),
-//   3072->768 71 us (81); M = 4096 1600->4800 107 us (138); M = 2048
-//   1600->1600 35 us (41);
-// * below that, 64 x 64 tiles on 8 waves (each 32 x 16): M = 2048 768->2304
-//   27.5 us (4 waves: 29.3), 3072->768 37 us (40);
-// * the int8 panels stay for M < 2048 at K < 1536, where the two time the same;
+// * the large tiles once they hold >= 144 of 128 x 128: M = 1280 768->3072
+//   13.9 us (int8 panels 19.2), 768->2304 13.0 (15.2), M = 512 1600->4800 20.5
+//   (25.9), M = 2560 1600->1600 26 (64 x 64 tiles 36); below, M = 1280 768->768
+//   11.7 (64 x 64 tiles 7.7);
+// * below that, 64 x 64 tiles on 8 waves (each 32 x 16) for M >= 2048 at
+//   K < 1536: M = 2048 768->768; the int8 panels elsewhere;
 // * at K >= 1536 the 64 x 64 tiles keep a 4-stage ring (two chunks of 32 in
 //   flight): M = 1024 3072->768 25.3 us against 31.5 with 3 stages, which time
 //   the same or better at K = 768 (6 stages: slower everywhere).
-bool f16_gemm_large(int m, int n, int k) {
-  const int64_t tiles = int64_t((m + 127) / 128) * ((n + 127) / 128);
-  return tiles >= 384 || (k >= 1536 && tiles >= 192);
-}
-bool f16_gemm_preferred(int m, int n, int k) { return f16_gemm_large(m, n, k) || (m >= 2048 && k < 1536); }
+bool f16_gemm_large(int m, int n) { return tiles_of(m, n, 128, 128) >= 144; }
+bool f16_gemm_preferred(int m, int n, int k) { return f16_gemm_large(m, n) || (m >= 2048 && k < 1536); }
 
-// Larger tiles halve the LDS bytes per MFMA (a wave's 128 x 64 or 128 x 32
-// block reads 12 / 10 KiB per 32 / 16 MFMAs, against 6 KiB per 8 for 64 x 32)
-// but hold one (256 x 256: 96 KiB, 202 registers) or two (256 x 128) 8-wave
-// workgroups per CU, so they win only where the grid fills whole rounds of
-// them (timed on MI355X, XL shapes, graph replays):
-// * 256 x 256 at K >= 4096 when the tiles make one nearly full round:
-//   M = 8192 6400->1600 (224 tiles) 199 us against 256; at 112 tiles 188
-//   against 143, at 294 (two rounds) 388 against 328;
-// * 256 x 128 from four rounds of two per CU at K < 4096: M = 8192
-//   1600->4800 180 against 194 us, 1600->6400 244 against 257, M = 10752
-//   1600->4800 238 against 250, 1600->6400 310 against 326; at 1.2-2 rounds
-//   slower (M = 4096 1600->4800 121 against 110 us).  Its occupancy (two
-//   8-wave workgroups per CU) needs <= 128 registers, held by the launch
-//   bound (a few epilogue values spill).
 hipError_t launch_f16(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* deferred) {
-  if (f16_gemm_large(g.m, g.n, g.k)) {
-    const int64_t cus = device_cus(), rows256 = (g.m + 255) / 256;
-    const int64_t t256 = rows256 * ((g.n + 255) / 256), t256x128 = rows256 * ((g.n + 127) / 128);
-    if (g.k >= 4096 && 4 * t256 >= 3 * cus && t256 <= cus) return launch_f16_cfg<2, 4, 8, 4, 3, 8, 2>(g, s, stream, deferred);
-    if (g.k < 4096 && t256x128 >= 4 * cus) return launch_f16_cfg<2, 4, 8, 2, 3, 8, 4>(g, s, stream, deferred);
-    return launch_f16_cfg<2, 4, 4, 2, 3, 4, 3>(g, s, stream, deferred);
-  }
+  if (f16_gemm_large(g.m, g.n) && g.lda <= (1 << 22)) return launch_tile<TW_REC16>(g, stream);
   if (g.k >= 1536) return launch_f16_cfg<2, 4, 2, 1, 4, 1, 3>(g, s, stream, deferred);
   return launch_f16_cfg<2, 4, 2, 1, 3, 1, 3>(g, s, stream, deferred);
 }
@@ -3068,6 +3505,10 @@ hipError_t gemm(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* de
       if (e != hipErrorNotSupported) return e;
     }
     return launch_panel(g, s, stream, deferred);
+  }
+  if (wvec && avec) {
+    const hipError_t e = g.w_int8 ? launch_row_tiles<TW_ROW8>(g, stream) : launch_row_tiles<TW_ROW16>(g, stream);
+    if (e != hipErrorNotSupported) return e;
   }
   if (g.m <= kRowMaxM && g.w_int8 && wvec && avec && s && s->queue_pool && !deferred) {
     const hipError_t e = g.m <= 16 ? launch_rowgemv(g, stream) : launch_rowgemm(g, stream);
