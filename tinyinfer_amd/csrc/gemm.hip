@@ -147,6 +147,14 @@ __device__ __forceinline__ void qkv_store_bt(const Epilogue& e, int b, int t, in
   }
 }
 
+// Cache element of head 0, dim 0 of EPI_QKV row m, or -1 for a padding row.
+__device__ __forceinline__ int64_t qkv_row_position(const Epilogue& e, int m) {
+  int b, t;
+  qkv_row(e, m, b, t);
+  if (t >= e.qlens[b]) return -1;
+  return ((int64_t(e.slots[b]) * e.layers + e.layer) * e.heads * e.capacity + int64_t(e.offsets[b]) + t) * 64;
+}
+
 __device__ __forceinline__ void qkv_store(const Epilogue& e, int m, int n, float val) {
   int b, t;
   qkv_row(e, m, b, t);
@@ -1499,10 +1507,12 @@ __device__ __forceinline__ void load_bias4(const Epilogue& e, int col, int n, co
 // any result is computed; a group of 4 columns inside the matrix goes out as
 // one 8-byte (fp16) or 16-byte (fp32) store when the layout allows it.
 // partials != null: the raw sums go to partials[(split m + row) n + col]
-// (split-K or a deferred finisher) instead.
+// (split-K or a deferred finisher) instead.  kv_at (EPI_QKV): the cache
+// position of each tile row (qkv_row_position), in LDS.
 template <int TR, int BN, int NT>
 __device__ __forceinline__ void tile_epilogue(const Epilogue& e, const float* ctile, int r0, int n0, int m, int n,
-                                              const float (&bias)[4], float* partials, int split) {
+                                              const float (&bias)[4], float* partials, int split,
+                                              const int64_t* kv_at = nullptr) {
   constexpr int CG = BN / 4, RS = NT / CG, RPT = TR / RS;
   static_assert(NT % CG == 0 && TR % RS == 0 && RPT >= 1, "whole row groups per thread");
   const int c4 = int(threadIdx.x) % CG, rl0 = int(threadIdx.x) / CG;
@@ -1556,6 +1566,18 @@ __device__ __forceinline__ void tile_epilogue(const Epilogue& e, const float* ct
         const int row = row_of(i);
         if (row >= m) break;
         const float4_t v = sums(i);
+        if (kv_at && vec) {
+          const half4_t h4 = {f16r(v[0] + bias[0]), f16r(v[1] + bias[1]), f16r(v[2] + bias[2]), f16r(v[3] + bias[3])};
+          *reinterpret_cast<half4_t*>(y + int64_t(row) * e.ldy + col) = h4;
+          const int64_t at = kv_at[rl0 + i * RS];
+          if (col >= e.hidden && at >= 0) {
+            const int part = col >= 2 * e.hidden ? 2 : 1;
+            const int c = col - part * e.hidden;
+            *reinterpret_cast<half4_t*>((part == 1 ? e.kcache : e.vcache) + at + int64_t(c >> 6) * e.capacity * 64 +
+                                        (c & 63)) = h4;
+          }
+          continue;
+        }
         int rb, rt;
         qkv_row(e, row, rb, rt);
         if (!vec) {
@@ -2906,6 +2928,13 @@ struct TileParams {
 // chunk.  M = 8192, 1600->6400, int8: 207 us; groups of 2 / 4: 235 / 213.
 constexpr int kTileGroup = 8;
 
+// LDS of a tile's operand rings, or of its epilogue's fp32 tile if larger.
+template <int TW, int BM, int BN, int EP>
+constexpr size_t tile_lds_ring() {
+  constexpr size_t ring = size_t(2) * BM * 128 + size_t(TW == TW_REC16 ? 2 : 3) * BN * 128;
+  return TW == TW_REC16 ? std::max(ring, size_t(BM / EP) * tile_pitch(BN) * 4) : ring;
+}
+
 // Tile (WM * MT * 16) x (WN * R * 16), WM x WN waves of MT x R MFMA blocks,
 // every output summed over K in 32-row MFMA steps from 0 upward whatever the
 // tile (so tile choices agree bit for bit).  What bounds it is keeping the
@@ -2941,8 +2970,11 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
   constexpr int UN = BN * 2 / NT;                   // row-major W: 8 x 4 units per thread and chunk
   static_assert(BM % (8 * W) == 0 && MT % 2 == 0, "whole A loads per wave, two halves of A blocks");
   static_assert(REC ? BN % (8 * W) == 0 : (UN >= 1 && BN * 2 % NT == 0 && R == 4), "W loads split evenly");
-  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];  // 2 A stages, SB W stages
+  // 2 A stages, SB W stages (the epilogue's tile reuses them), and for records
+  // the cache position of each row of an EPI_QKV tile.
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   uint8_t* const blds = lds + 2 * ASTAGE;
+  int64_t* const kv_at = reinterpret_cast<int64_t*>(lds + tile_lds_ring<TW, BM, BN, EP>());
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
@@ -3171,7 +3203,13 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
   }
 
   if constexpr (REC) {
-    // Through an LDS fp32 tile of BM / EP rows x BN, EP passes.
+    // Through an LDS fp32 tile of BM / EP rows x BN, EP passes.  A QKV tile's
+    // cache positions (a search of row_start and three dependent loads each)
+    // are found once per row here, not by every thread for each of its rows:
+    // M = 2560, 1600->4800 80 -> 52 us.
+    const bool qkv = p.epi.kind == EPI_QKV;
+    if (qkv && int(threadIdx.x) < BM)
+      kv_at[threadIdx.x] = m0 + int(threadIdx.x) < p.m ? qkv_row_position(p.epi, m0 + int(threadIdx.x)) : -1;
     float bias[4];
     load_bias4(p.epi, n0 + 4 * int(threadIdx.x % (BN / 4)), p.n, p.a, bias);
     constexpr int PR = BM / EP;
@@ -3191,7 +3229,8 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
             ctile[(rb + 4 * g + v) * tile_pitch(BN) + (wn * R + r) * 16 + j] = acc[t][r][v];
       }
       __syncthreads();
-      tile_epilogue<PR, BN, NT>(p.epi, ctile, m0 + pass * PR, n0, p.m, p.n, bias, nullptr, 0);
+      tile_epilogue<PR, BN, NT>(p.epi, ctile, m0 + pass * PR, n0, p.m, p.n, bias, nullptr, 0,
+                                qkv ? kv_at + pass * PR : nullptr);
     }
   } else {
     // Lane (j, g): rows 4g + v of each block, columns 4j .. 4j + 3 of the wave's 64.
@@ -3245,8 +3284,8 @@ template <int TW, int WM, int WN, int MT, int R, int EP, int OCC>
 hipError_t launch_tile_cfg(const GemmArgs& g, int m_begin, int m_end, hipStream_t stream) {
   constexpr int BM = WM * MT * 16, BN = WN * R * 16;
   constexpr bool REC = TW == TW_REC16;
-  constexpr size_t kRing = size_t(2) * BM * 128 + size_t(REC ? 2 : 3) * BN * 128;
-  constexpr size_t kLds = std::max(kRing, REC ? size_t(BM / EP) * tile_pitch(BN) * 4 : size_t(0));
+  constexpr size_t kLds = tile_lds_ring<TW, BM, BN, EP>() + (REC ? BM * sizeof(int64_t) : 0);
+  static_assert(!REC || WM * WN * 64 >= BM, "a thread per tile row finds its cache position");
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
   if (attr != hipSuccess) return attr;
