@@ -612,6 +612,31 @@ def test_row_major_large_tiles_fused(ops, m, n, k):
         assert bool(((y.double() - gelu).abs() <= 2.0 ** -11 * gelu.abs() + 1e-6 * z.abs() + 2.0 ** -24).all())
 
 
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 4, 8), (1, 5, 40), (3, 7, 768), (16, 65, 104), (16, 1001, 1600), (5, 13003, 72),     # up to 16 rows
+    (17, 6, 8), (32, 129, 3072), (33, 63, 200), (32, 12999, 136), (64, 1003, 768),           # 16- and 32-row blocks
+    (65, 77, 1000), (130, 2301, 768), (1000, 333, 400), (512, 768, 3072), (200, 1600, 64),   # K splits
+])
+def test_row_major_any_alignment(ops, m, n, k, int8):
+    """Row kernels over weights whose rows start anywhere, at each offset of the
+    first byte (int8) or element (fp16), against 64-bit sums.  The matrix's
+    neighbours in memory are NaN (fp16) or -128 (int8): a column or row taken
+    from them shows."""
+    t = torch()
+    say("row-major any alignment", m, n, k, int8)
+    a, q, s, w, bias = large_operands(m, n, k, m + n + k)
+    ref, bound = large_reference(a, w, bias)
+    for off in range(4 if int8 else 2):
+        src, fill = (q, -128) if int8 else (w, float("nan"))
+        store = t.full((n * k + 64,), fill, dtype=src.dtype, device="cuda")
+        held = store[32 + off:32 + off + n * k].view(k, n)
+        held.copy_(src)
+        out = (ops.gemm_int8(a, held, s, bias=bias, output_dtype=t.float32) if int8
+               else ops.gemm(a, held, bias=bias, output_dtype=t.float32))
+        assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(1100, 2050, 96), (3601, 3841, 160), (5000, 3844, 32), (1100, 2050, 64)])
 def test_record_large_tiles(ops, m, n, k):
     """fp16 records: the value of every tile choice, and the bits of the

@@ -11,8 +11,8 @@
 //    takes the part-block kernel instead when the caller does not batch rows
 //    (standalone GEMV calls): no MFMA, 8 columns per workgroup, twice the
 //    workgroups of the 16-column MFMA blocks.
-//  * row GEMV / GEMM (M <= 1024, row-major weights of the C ABIs, aligned
-//    operands): about 192 workgroups, each one 64-column tile of 16 (M <= 64)
+//  * row GEMV / GEMM (M <= 1024, row-major weights of the C ABIs of either type
+//    and any alignment, 16-byte rows of A): about 192 workgroups, each one 64-column tile of 16 (M <= 64)
 //    or 32 rows over a range of 32-row K steps, every load of a wave's round
 //    in flight at once, the skinny kernel's fragments and MFMAs; K splits
 //    finish in the launch through the queue pool (rowgemv_kernel at M <= 16,
@@ -210,6 +210,13 @@ __device__ __forceinline__ void apply_epilogue(const Epilogue& e, int m, int n, 
 // ---------------------------------------------------------------------------
 // Skinny kernel
 // ---------------------------------------------------------------------------
+// Workgroup id -> its place when each of the 8 XCDs (workgroups go to them
+// round-robin) takes one contiguous run of places.
+__device__ __forceinline__ int xcd_run_id(int id, int n) {
+  const int x = id & 7;
+  return x * (n >> 3) + min(x, n & 7) + (id >> 3);
+}
+
 struct SkinnyParams {
   const uint16_t* a;
   int64_t lda;
@@ -278,6 +285,80 @@ __device__ __forceinline__ void load_wfrag(WFrag<INT8>& f, const void* w, int K,
       f.d[2 * r] = v0;
       f.d[2 * r + 1] = v1;
     }
+  }
+}
+
+// Two dwords at a dword-aligned address.
+struct __attribute__((packed, aligned(4))) PairDwords {
+  uint2 v;
+  __device__ __forceinline__ operator uint2() const { return v; }
+};
+
+// The same for rows that start at any byte (int8) or any element (fp16) of N >= 4
+// columns and K a multiple of 8; the last columns are loaded from column N - 4, those below col
+// shifted out.  fp16: the four columns in one load as they lie.  int8: the two
+// aligned dwords around them (a misaligned dword load costs twice an aligned
+// pair: 52 against 27 us for the tied head, 768 x 50257 at M = 32), which a
+// first or last row of the matrix would take from outside it: those load
+// exactly their four bytes.
+template <bool INT8>
+__device__ __forceinline__ void load_wfrag_any(WFrag<INT8>& f, const void* w, int K, int N, int64_t LDW, int krow,
+                                               int col) {
+  constexpr int B = INT8 ? 1 : 2;
+  const int from = min(col, N - 4), drop = min(col - from, 4) * 8 * B;
+  const char* p = static_cast<const char*>(w) + (int64_t(krow) * LDW + from) * B;
+  if constexpr (INT8) {
+    if (krow > 0 && krow + 8 < K) {
+      uint2 v[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const char* at = p + int64_t(r) * LDW;
+        v[r] = *reinterpret_cast<const PairDwords*>(at - (reinterpret_cast<uintptr_t>(at) & 3));
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const uint32_t by = uint32_t(reinterpret_cast<uintptr_t>(p) + uintptr_t(r) * uintptr_t(LDW)) & 3u;
+        f.d[r] = __builtin_amdgcn_alignbyte(v[r].y, v[r].x, by);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        f.d[r] = 0;
+        if (krow + r < K) __builtin_memcpy(&f.d[r], p + int64_t(r) * LDW, 4);
+      }
+    }
+    if (drop) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f.d[r] = drop < 32 ? f.d[r] >> drop : 0;
+    }
+  } else {
+    uint64_t v[8] = {};
+    if (krow < K) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) __builtin_memcpy(&v[r], p + int64_t(r) * LDW * 2, 8);
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      if (drop) v[r] = drop < 64 ? v[r] >> drop : 0;
+      f.d[2 * r] = uint32_t(v[r]);
+      f.d[2 * r + 1] = uint32_t(v[r] >> 32);
+    }
+  }
+}
+
+// And for rows of whole aligned 4-column groups (K a multiple of 8): columns
+// past N come from the last group, whose outputs past N are not stored.
+template <bool INT8>
+__device__ __forceinline__ void load_wfrag_row(WFrag<INT8>& f, const void* w, int K, int N, int64_t LDW, int krow,
+                                               int col) {
+  constexpr int B = INT8 ? 1 : 2;
+  const char* p = static_cast<const char*>(w) + (int64_t(krow) * LDW + min(col, (N + 3) / 4 * 4 - 4)) * B;
+  if (krow < K) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) __builtin_memcpy(&f.d[r * B], __builtin_assume_aligned(p + int64_t(r) * LDW * B, 4 * B), 4 * B);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 8 * B; ++r) f.d[r] = 0;
   }
 }
 
@@ -462,7 +543,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_kernel(SkinnyParams p) 
   }
 }
 
-// Row-major int8 GEMV of the C ABIs at M <= 16 (q [K][N] as the reference
+// Row-major GEMV of the C ABIs at M <= 16 (int8 or fp16 [K][N] as the reference
 // keeps it, reference kernels/src/cuda/tc/gemm.cu:21): workgroup (tile, split)
 // covers one 64-column tile over at most W * S 32-row K steps; wave w takes
 // steps w, w + W, ... with every load of the wave in flight before its first
@@ -472,28 +553,28 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_kernel(SkinnyParams p) 
 // them in split order (one round of loads) and runs it.  The plan depends on N
 // and K only, so a row's result does not depend on M.
 constexpr int kRowSplits = 16;
-template <int W, int S>
+template <bool INT8, bool WVEC, int W, int S>
 __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
   __shared__ float red[W][16][65];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 15, g = lane >> 4;
   // Consecutive (tile, split) ids per XCD (blocks go round-robin over the 8
   // XCDs): the two tiles that share a 128-byte weight line read it through one L2.
-  const int nb = gridDim.x, bid = blockIdx.x;
-  const int logical = (nb % 8 == 0) ? (bid % 8) * (nb / 8) + bid / 8 : bid;
+  const int logical = xcd_run_id(int(blockIdx.x), int(gridDim.x));
   const int tile = logical % p.ntile, split = logical / p.ntile;
   const int s0 = split * p.steps_per_block, s1 = min(p.steps, s0 + p.steps_per_block);
   const int n0 = tile * 64, col = n0 + 4 * j;
   float sc[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) sc[c] = col + c < p.n ? p.scales[col + c] : 0.f;
-  WFrag<true> f[S];
+  for (int c = 0; c < 4; ++c) sc[c] = INT8 && col + c < p.n ? p.scales[col + c] : 0.f;
+  WFrag<INT8> f[S];
   half8_t a[S];
 #pragma unroll
   for (int i = 0; i < S; ++i) {
     const int st = s0 + wave + W * i;
     if (st < s1) {
-      load_wfrag<true, true>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
+      if constexpr (WVEC) load_wfrag_row<INT8>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
+      else load_wfrag_any<INT8>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
       a[i] = afrag<true>(p.a, p.lda, p.m, p.k, j, st * 32 + 8 * g);
     }
   }
@@ -505,7 +586,7 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
     if (s0 + wave + W * i < s1) {
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bfrag<true>(f[i], c, sc[c]), acc[c], 0, 0, 0);
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], bfrag<INT8>(f[i], c, sc[c]), acc[c], 0, 0, 0);
     }
   }
   // MFMA output: lane holds rows 4g + v (v = 0..3) of column j of each 16x16 block.
@@ -546,7 +627,7 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
   depart(slot.ctr + tile * kCounterStride);
 }
 
-// Row-major int8 GEMM of the C ABIs at 16 < M <= 1024 (q [K][N] as the reference
+// Row-major GEMM of the C ABIs at 16 < M <= 1024 (int8 or fp16 [K][N] as the reference
 // keeps it, reference kernels/src/cuda/tc/gemm.cu:21), built like the skinny
 // kernel (weight fragments from HBM straight into MFMA B registers, dequantised
 // there, no LDS staging): workgroup (tile, row block, split) covers one
@@ -558,8 +639,10 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
 // order (one round of loads) and runs it.  Row blocks are 16 rows up to M = 64,
 // then 32; the K split follows the count of (tile, row block) units, so unlike
 // the M <= 16 GEMV a row's sums may differ between M values (the reference ABI
-// promises no batch invariance; the runtime never takes this path).
-template <int MT, int W, int S>
+// promises no batch invariance; the runtime never takes this path).  fp16 weights
+// (before, the skinny and tiled kernels): M = 512 3072->768 35 -> 17 us; the tied
+// head at M = 32: int8 52 -> 20 us (2.2 TB/s), fp16 84 -> 31 us.
+template <bool INT8, bool WVEC, int MT, int W, int S>
 __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   constexpr int R = 16 * MT, NT = W * 64;
   constexpr int OUT4 = (R * 16 + NT - 1) / NT;  // float4 outputs of a finishing thread
@@ -570,8 +653,7 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   // Consecutive ids per XCD (blocks go round-robin over the 8 XCDs), column
   // tile fastest: the two tiles that share a 128-byte weight line, and the
   // tiles that share a row block's A rows, are read through one L2.
-  const int nb = gridDim.x, bid = blockIdx.x;
-  const int logical = (nb % 8 == 0) ? (bid % 8) * (nb / 8) + bid / 8 : bid;
+  const int logical = xcd_run_id(int(blockIdx.x), int(gridDim.x));
   const int tile = logical % p.ntile, rest = logical / p.ntile;
   const int rb = rest % p.rblocks, split = rest / p.rblocks;
   const int m0 = rb * R, rows = min(R, p.m - m0);
@@ -579,20 +661,21 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   const int n0 = tile * 64, col = n0 + 4 * j;
   float sc[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) sc[c] = col + c < p.n ? p.scales[col + c] : 0.f;
+  for (int c = 0; c < 4; ++c) sc[c] = INT8 && col + c < p.n ? p.scales[col + c] : 0.f;
   float4_t acc[MT][4];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[t][c] = float4_t{0.f, 0.f, 0.f, 0.f};
   for (int base = s0 + wave; base < s1; base += W * S) {
-    WFrag<true> f[S];
+    WFrag<INT8> f[S];
     half8_t a[S][MT];
 #pragma unroll
     for (int i = 0; i < S; ++i) {
       const int st = base + W * i;
       if (st < s1) {
-        load_wfrag<true, true>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
+        if constexpr (WVEC) load_wfrag_row<INT8>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
+        else load_wfrag_any<INT8>(f[i], p.w, p.k, p.n, p.ldw, st * 32 + 8 * g, col);
 #pragma unroll
         for (int t = 0; t < MT; ++t) a[i][t] = afrag<true>(p.a, p.lda, p.m, p.k, m0 + 16 * t + j, st * 32 + 8 * g);
       }
@@ -602,7 +685,7 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
       if (base + W * i < s1) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const half8_t b = bfrag<true>(f[i], c, sc[c]);
+          const half8_t b = bfrag<INT8>(f[i], c, sc[c]);
 #pragma unroll
           for (int t = 0; t < MT; ++t) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][t], b, acc[t][c], 0, 0, 0);
         }
@@ -2221,11 +2304,12 @@ int skinny_splits(int m, int n, int k, size_t capacity) {
 // than kRowSplits splits, or partials beyond the pool): the caller then takes
 // the skinny kernel.
 constexpr int kRowTargetBlocks = 192;
-template <int W, int S>
+template <bool INT8, bool WVEC, int W, int S>
 hipError_t launch_rowgemv_ws(const SkinnyParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((rowgemv_kernel<W, S>), dim3(unsigned(p.ntile) * unsigned(p.splits)), dim3(W * 64), 0, stream, p);
+  hipLaunchKernelGGL((rowgemv_kernel<INT8, WVEC, W, S>), dim3(unsigned(p.ntile) * unsigned(p.splits)), dim3(W * 64), 0, stream, p);
   return hipGetLastError();
 }
+template <bool INT8, bool WVEC>
 hipError_t launch_rowgemv(const GemmArgs& g, hipStream_t stream) {
   SkinnyParams p{};
   p.a = g.a; p.lda = g.lda; p.w = g.w; p.scales = g.scales;
@@ -2243,10 +2327,10 @@ hipError_t launch_rowgemv(const GemmArgs& g, hipStream_t stream) {
   p.steps_per_block = spb;
   p.splits = splits;
   p.pool = splits > 1;
-  if (spb <= 8) return launch_rowgemv_ws<8, 1>(p, stream);
-  if (spb <= 16) return launch_rowgemv_ws<16, 1>(p, stream);
-  if (spb <= 32) return launch_rowgemv_ws<16, 2>(p, stream);
-  return launch_rowgemv_ws<16, 4>(p, stream);
+  if (spb <= 8) return launch_rowgemv_ws<INT8, WVEC, 8, 1>(p, stream);
+  if (spb <= 16) return launch_rowgemv_ws<INT8, WVEC, 16, 1>(p, stream);
+  if (spb <= 32) return launch_rowgemv_ws<INT8, WVEC, 16, 2>(p, stream);
+  return launch_rowgemv_ws<INT8, WVEC, 16, 4>(p, stream);
 }
 
 // Plan of rowgemm_kernel (16 < M <= kRowMaxM): rows in blocks of 16 up to
@@ -2258,12 +2342,13 @@ hipError_t launch_rowgemv(const GemmArgs& g, hipStream_t stream) {
 // of 16-row blocks has more than 8 steps; S steps a round, rounds repeated
 // over longer splits.
 constexpr int kRowMaxM = 1024;
-template <int MT, int W, int S>
+template <bool INT8, bool WVEC, int MT, int W, int S>
 hipError_t launch_rowgemm_ws(const SkinnyParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((rowgemm_kernel<MT, W, S>), dim3(unsigned(p.ntile * p.rblocks * p.splits)), dim3(W * 64), 0,
+  hipLaunchKernelGGL((rowgemm_kernel<INT8, WVEC, MT, W, S>), dim3(unsigned(p.ntile * p.rblocks * p.splits)), dim3(W * 64), 0,
                      stream, p);
   return hipGetLastError();
 }
+template <bool INT8, bool WVEC>
 hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   SkinnyParams p{};
   p.a = g.a; p.lda = g.lda; p.w = g.w; p.scales = g.scales;
@@ -2271,7 +2356,9 @@ hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   p.ldw = g.ldw > 0 ? g.ldw : g.n;
   p.ntile = (g.n + 63) / 64;
   p.steps = (g.k + 31) / 32;
-  const int mt = g.m <= 64 ? 1 : 2;
+  // (A 16-row block would read the weights once per block; once the column
+  // tiles alone fill the chip, 32 rows share them.)
+  const int mt = g.m <= 64 && p.ntile < kRowTargetBlocks ? 1 : 2;
   p.rblocks = (g.m + 16 * mt - 1) / (16 * mt);
   const int64_t units = int64_t(p.ntile) * p.rblocks;
   int splits = int(std::clamp<int64_t>((kRowTargetBlocks + units / 2) / units, 1, rowgemm_max_splits(mt, 8)));
@@ -2284,16 +2371,20 @@ hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   p.splits = splits;
   p.pool = splits > 1;
   if (mt == 1) {
-    if (spb <= 8) return launch_rowgemm_ws<1, 8, 1>(p, stream);
-    if (spb <= 16) return launch_rowgemm_ws<1, 16, 1>(p, stream);
-    if (spb <= 32) return launch_rowgemm_ws<1, 16, 2>(p, stream);
-    return launch_rowgemm_ws<1, 16, 4>(p, stream);
+    if (spb <= 8) return launch_rowgemm_ws<INT8, WVEC, 1, 8, 1>(p, stream);
+    if (spb <= 16) return launch_rowgemm_ws<INT8, WVEC, 1, 16, 1>(p, stream);
+    if (spb <= 32) return launch_rowgemm_ws<INT8, WVEC, 1, 16, 2>(p, stream);
+    return launch_rowgemm_ws<INT8, WVEC, 1, 16, 4>(p, stream);
   }
-  if (spb <= 8) return launch_rowgemm_ws<2, 8, 1>(p, stream);
-  if (spb <= 16) return launch_rowgemm_ws<2, 8, 2>(p, stream);
-  return launch_rowgemm_ws<2, 8, 4>(p, stream);
+  if (spb <= 8) return launch_rowgemm_ws<INT8, WVEC, 2, 8, 1>(p, stream);
+  if (spb <= 16) return launch_rowgemm_ws<INT8, WVEC, 2, 8, 2>(p, stream);
+  return launch_rowgemm_ws<INT8, WVEC, 2, 8, 4>(p, stream);
 }
 
+template <bool INT8, bool WVEC>
+hipError_t launch_row(const GemmArgs& g, hipStream_t stream) {
+  return g.m <= 16 ? launch_rowgemv<INT8, WVEC>(g, stream) : launch_rowgemm<INT8, WVEC>(g, stream);
+}
 
 // The skinny finisher spreads a tile's splits over its idle threads: rows
 // below M of each 16-row pass take 16 threads each, and the 256 threads form
@@ -2983,8 +3074,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
   // tiles, walked in groups of kTileGroup tile rows, column by column.
   int tm, tn;
   {
-    const int nbk = int(gridDim.x), bid = int(blockIdx.x), q = nbk >> 3, rem = nbk & 7, x = bid & 7;
-    const int tile = x * q + min(x, rem) + (bid >> 3);
+    const int tile = xcd_run_id(int(blockIdx.x), int(gridDim.x));
     const int tiles_m = p.tiles / p.tiles_n;
     const int per_group = kTileGroup * p.tiles_n, group = tile / per_group, first = group * kTileGroup;
     const int gm = min(tiles_m - first, kTileGroup), r = tile - group * per_group;
@@ -3356,13 +3446,13 @@ hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
 // Row-major weights over the large tiles, for operands that allow their wide
 // loads.  hipErrorNotSupported: the shape is better served by the kernels that
 // split K over few tiles (us, this kernel against them):
-// * int8 up to kRowMaxM rows (the row GEMM): from 160 tiles of 64 x 128:
-//   512 x 768 x 3072 12.4 / 14.9, 1024 x 1600 x 1600 21.5 / 25.2, 1024 x 768 x
-//   3072 15.1 / 25.8; below, 1024 x 768 x 768 12.1 / 9.8, 512 x 3072 x 768
-//   36 / 14.8; the longest K keeps the row GEMM up to 160 tiles of 128 x 128
+// * up to kRowMaxM rows (the row GEMM): from 160 tiles of 64 x 128: 512 x 768 x
+//   3072 12.4 / 14.9, 1024 x 1600 x 1600 21.5 / 25.2, 1024 x 768 x 3072 15.1 /
+//   25.8; below, 1024 x 768 x 768 12.1 / 9.8, 512 x 3072 x 768 36 / 14.8 (fp16 34 /
+//   17); the longest K keeps the row GEMM up to 144 tiles of 128 x 128
 //   (1024 x 6400 x 1600 87 / 83);
-// * fp16 (the tiled kernel): from 100 tiles of 64 x 64: 256 x 768 x 3072 9.9 /
-//   14.2, 1024 x 3072 x 768 37 / 62; below, 128 x 768 x 768 9.6 / 8.7.
+// * above, the tiled kernel only where K is no multiple of 8: 1500 x 768 x 768
+//   12.1 / 16.4, 1500 x 3072 x 768 44 / 64.
 template <int TW>
 hipError_t launch_row_tiles(const GemmArgs& g, hipStream_t stream) {
   const int64_t ldw = g.ldw > 0 ? g.ldw : g.n;
@@ -3370,13 +3460,9 @@ hipError_t launch_row_tiles(const GemmArgs& g, hipStream_t stream) {
     return hipErrorNotSupported;
   const int64_t mid = tiles_of(g.m, g.n, 128, 128);
   if (mid >= 144) return launch_tile<TW>(g, stream);
-  if constexpr (TW == TW_ROW8) {
-    if (g.m <= kRowMaxM && (tiles_of(g.m, g.n, 64, 128) < 160 || g.k > 4096)) return hipErrorNotSupported;
-    return launch_tile_cfg<TW, 2, 2, 2, 4, 2, 2>(g, 0, g.m, stream);
-  } else {
-    if (tiles_of(g.m, g.n, 64, 64) < 100) return hipErrorNotSupported;
-    return launch_tile_cfg<TW, 2, 1, 2, 4, 2, 2>(g, 0, g.m, stream);
-  }
+  if (g.m <= kRowMaxM && (tiles_of(g.m, g.n, 64, 128) < 160 || g.k > 4096)) return hipErrorNotSupported;
+  return TW == TW_ROW8 ? launch_tile_cfg<TW, 2, 2, 2, 4, 2, 2>(g, 0, g.m, stream)
+                       : launch_tile_cfg<TW, 2, 1, 2, 4, 2, 2>(g, 0, g.m, stream);
 }
 
 // Tile choice over the fp16 records, and when they beat the int8 panel
@@ -3549,8 +3635,12 @@ hipError_t gemm(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* de
     const hipError_t e = g.w_int8 ? launch_row_tiles<TW_ROW8>(g, stream) : launch_row_tiles<TW_ROW16>(g, stream);
     if (e != hipErrorNotSupported) return e;
   }
-  if (g.m <= kRowMaxM && g.w_int8 && wvec && avec && s && s->queue_pool && !deferred) {
-    const hipError_t e = g.m <= 16 ? launch_rowgemv(g, stream) : launch_rowgemm(g, stream);
+  // (fp16 rows of no whole 4-column groups, over columns that fill the chip by
+  // themselves: the tiled kernel from 33 rows, M = 64 768 x 50257 51 against 55 us.)
+  const bool tiled_fp16 = !g.w_int8 && !wvec && g.m > 32 && g.n >= 64 * kRowTargetBlocks;
+  if (g.m <= kRowMaxM && g.n >= 4 && avec && g.k % 8 == 0 && s && s->queue_pool && !deferred && !tiled_fp16) {
+    const hipError_t e = g.w_int8 ? (wvec ? launch_row<true, true>(g, stream) : launch_row<true, false>(g, stream))
+                                  : (wvec ? launch_row<false, true>(g, stream) : launch_row<false, false>(g, stream));
     if (e != hipErrorNotSupported) return e;
   }
   if (g.m <= 16) return g.w_int8 ? launch_skinny<true, 1>(g, wvec, avec, s, stream, deferred)
