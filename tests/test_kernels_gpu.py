@@ -1122,6 +1122,34 @@ def test_non_default_stream_and_input_lifetime(ops):
     close(host(actual), expected)
 
 
+@pytest.mark.parametrize("batch,heads,nq,nk,d,causal", [
+    (1, 1, 2, 2, 64, True), (1, 3, 65, 70, 128, True), (3, 3, 130, 130, 64, True),     # rows no multiple of 8
+    (8, 25, 200, 256, 64, True), (5, 13, 129, 300, 128, False), (3, 33, 1000, 1000, 64, True),
+])
+def test_prefill_attention_every_row_and_tile(ops, batch, heads, nq, nk, d, causal):
+    """Each (b, h) row and query tile is taken once, whatever the row count, with
+    ragged lengths; padded queries are exactly zero.  fp16 probabilities and
+    output: 2^-10 of sum p |v| around the 64-bit result."""
+    t = torch()
+    say("prefill rows", batch, heads, nq, nk, d, causal)
+    gen = t.Generator(device="cuda").manual_seed(batch + heads + nq)
+    q, k, v = (t.randn(batch, heads, n, d, generator=gen, device="cuda").half() for n in (nq, nk, nk))
+    kl = [nk - (17 * b) % (nk // 2) for b in range(batch)]
+    ql = [min(nq - (5 * b) % (nq // 2), n) for b, n in enumerate(kl)]
+    off = [n - m for m, n in zip(ql, kl)]
+    out = ops.attention(q, k, v, q_lengths=ql, kv_lengths=kl, query_offsets=off, causal=causal).double()
+    for b in range(batch):
+        score = q[b, :, :ql[b]].double() @ k[b, :, :kl[b]].double().transpose(1, 2).contiguous() / d ** 0.5
+        if causal:
+            at = t.arange(ql[b], device="cuda")[:, None] + off[b]
+            score.masked_fill_(t.arange(kl[b], device="cuda")[None] > at, float("-inf"))
+        p = t.softmax(score, -1)
+        size = p @ v[b, :, :kl[b]].double().abs()
+        err = (out[b, :, :ql[b]] - p @ v[b, :, :kl[b]].double()).abs()
+        assert bool((err <= 2.0 ** -10 * size + 2.0 ** -24).all())
+        assert not out[b, :, ql[b]:].any()
+
+
 def test_attention_metadata_follows_the_stream(ops):
     """Back-to-back calls with other lengths, none waited for: each call's
     metadata reaches its own kernel (equal to the same call alone), and a call
