@@ -551,7 +551,9 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_kernel(SkinnyParams p) 
 // LDS; with one split the workgroup runs the epilogue, otherwise each split's
 // sums go to the queue's pool slot and the tile's last split to arrive adds
 // them in split order (one round of loads) and runs it.  The plan depends on N
-// and K only, so a row's result does not depend on M.
+// and K only, so a row's result does not depend on M.  fp16 weights (before, the
+// skinny kernel): M = 8 3072->768 9.0 -> 5.9 us; the tied head 768 x 50257, whose
+// rows start at any byte, at M = 4: 47 -> 18.5 us (int8).
 constexpr int kRowSplits = 16;
 template <bool INT8, bool WVEC, int W, int S>
 __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
