@@ -582,7 +582,12 @@ def test_row_major_large_tiles(ops, m, n, k, int8):
     out = call(a, bias=bias, output_dtype=t.float32)
     assert bool(((out.double() - ref).abs() <= bound).all())
     assert t.equal(call(a, bias=bias, config=6, output_dtype=t.float32), out)
-    assert t.equal(call(a, bias=bias), out.half())
+    # (Few rows or tiles take another kernel for fp32 outputs, so their sums may be
+    # ordered otherwise: half an fp16 step around the 64-bit bound.)
+    half = call(a, bias=bias).double()
+    assert bool(((half - ref).abs() <= bound + 2.0 ** -11 * (ref.abs() + bound) + 2.0 ** -25).all())
+    if m > 1024 and -(-m // 64) * -(-n // 64) >= 256:
+        assert t.equal(half, out.half().double())
     bad = a.clone()
     bad[m - 2, k - 1] = float("inf")
     got = call(bad, output_dtype=t.float32)

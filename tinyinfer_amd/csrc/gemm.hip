@@ -3455,6 +3455,36 @@ hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
   }
 }
 
+// Row-major W (the reference ABI's [K, N]).  Each K step of a workgroup waits
+// for one global round trip, so a grid of few tiles (M = 64, 3072 -> 768: 12
+// tiles x 96 steps, 138 us) splits K until >= 256 workgroups run (at least 4
+// steps each); the splits are summed in a fixed order and the epilogue applied
+// by the last workgroup of each tile (queue pool, capped split count) or by
+// splitk_epilogue_kernel over caller scratch.  Canonical (batch-invariant)
+// calls stay unsplit: their K order must not depend on M.
+// Split count of the row-major M > 32 kernel (0 capacity or a canonical call:
+// one split), after rounding to whole step ranges.
+int tiled_splits(int m, int n, int k, bool canonical, size_t capacity) {
+  const int steps = (k + TBK - 1) / TBK;
+  const int64_t tiles = int64_t((n + TBN - 1) / TBN) * ((m + TBM - 1) / TBM);
+  int splits = 1;
+  if (!canonical && capacity > 0 && tiles < 256) {
+    splits = int(std::min<int64_t>((256 + tiles - 1) / tiles, std::max(1, steps / 4)));
+    while (splits > 1 && size_t(splits) * m * n > capacity) --splits;
+  }
+  const int per = (steps + splits - 1) / splits;
+  return (steps + per - 1) / per;
+}
+
+int tiled_plan(const GemmArgs& g, const Scratch* s) {
+  const int steps = (g.k + TBK - 1) / TBK;
+  const int64_t tiles = int64_t((g.n + TBN - 1) / TBN) * ((g.m + TBM - 1) / TBM);
+  const bool pool = s && s->queue_pool && tiles <= kPoolTiles;
+  const int splits = tiled_splits(g.m, g.n, g.k, g.canonical,
+                                  pool ? kPoolFloats : (s && s->partials) ? s->partial_floats : 0);
+  return pool ? pool_splits(splits, tiles, TBM * TBN, kTileRounds * pool_max_splits(TBM / (256 / (TBN / 4))), steps) : splits;
+}
+
 // Row-major weights over the large tiles, for operands that allow their wide
 // loads.  hipErrorNotSupported: the shape is better served by the kernels that
 // split K over few tiles (us, this kernel against them):
@@ -3464,11 +3494,19 @@ hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
 //   17); the longest K keeps the row GEMM up to 144 tiles of 128 x 128
 //   (1024 x 6400 x 1600 87 / 83);
 // * above, the tiled kernel only where K is no multiple of 8: 1500 x 768 x 768
-//   12.1 / 16.4, 1500 x 3072 x 768 44 / 64.
+//   12.1 / 16.4, 1500 x 3072 x 768 44 / 64;
+// * fp32 outputs show the length of the sums that 16 bits hide, and here every
+//   one is a single chain over K: they stay with the kernels that cut K (the int8
+//   row GEMM up to kRowMaxM rows, the tiled kernel where it splits).  Distance
+//   from 64-bit sums, this kernel against them: 1024 x 768 x 3072 1.8e-7 / 8.7e-8
+//   (15.1 / 25.8 us), 1024 x 1600 x 6400 2.5e-7 / 1.1e-7.
 template <int TW>
-hipError_t launch_row_tiles(const GemmArgs& g, hipStream_t stream) {
+hipError_t launch_row_tiles(const GemmArgs& g, const Scratch* s, hipStream_t stream) {
   const int64_t ldw = g.ldw > 0 ? g.ldw : g.n;
   if (g.k % 8 != 0 || g.lda > (1 << 22) || ldw > (1 << 24) || g.epi.kind == EPI_QKV || g.epi.p32 || g.m <= 32)
+    return hipErrorNotSupported;
+  if ((g.epi.kind == EPI_F32 || g.epi.kind == EPI_RAW_F32) &&
+      ((TW == TW_ROW8 && g.m <= kRowMaxM) || tiled_plan(g, s) > 1))
     return hipErrorNotSupported;
   const int64_t mid = tiles_of(g.m, g.n, 128, 128);
   if (mid >= 144) return launch_tile<TW>(g, stream);
@@ -3497,39 +3535,15 @@ hipError_t launch_f16(const GemmArgs& g, const Scratch* s, hipStream_t stream, i
   return launch_f16_cfg<2, 4, 2, 1, 3, 1, 3>(g, s, stream, deferred);
 }
 
-// Row-major W (the reference ABI's [K, N]).  Each K step of a workgroup waits
-// for one global round trip, so a grid of few tiles (M = 64, 3072 -> 768: 12
-// tiles x 96 steps, 138 us) splits K until >= 256 workgroups run (at least 4
-// steps each); the splits are summed in a fixed order and the epilogue applied
-// by the last workgroup of each tile (queue pool, capped split count) or by
-// splitk_epilogue_kernel over caller scratch.  Canonical (batch-invariant)
-// calls stay unsplit: their K order must not depend on M.
-// Split count of the row-major M > 32 kernel (0 capacity or a canonical call:
-// one split), after rounding to whole step ranges.
-int tiled_splits(int m, int n, int k, bool canonical, size_t capacity) {
-  const int steps = (k + TBK - 1) / TBK;
-  const int64_t tiles = int64_t((n + TBN - 1) / TBN) * ((m + TBM - 1) / TBM);
-  int splits = 1;
-  if (!canonical && capacity > 0 && tiles < 256) {
-    splits = int(std::min<int64_t>((256 + tiles - 1) / tiles, std::max(1, steps / 4)));
-    while (splits > 1 && size_t(splits) * m * n > capacity) --splits;
-  }
-  const int per = (steps + splits - 1) / splits;
-  return (steps + per - 1) / per;
-}
-
 template <bool INT8>
 hipError_t launch_tiled(const GemmArgs& g, bool wvec, bool avec, const Scratch* s, hipStream_t stream) {
   TiledParams p{};
   p.a = g.a; p.lda = g.lda; p.w = g.w; p.scales = g.scales;
   p.m = g.m; p.n = g.n; p.k = g.k; p.epi = g.epi;
   p.ldw = g.ldw > 0 ? g.ldw : g.n;
-  const int steps = (g.k + TBK - 1) / TBK;
+  const int steps = (g.k + TBK - 1) / TBK, splits = tiled_plan(g, s);
   const int64_t tiles = int64_t((g.n + TBN - 1) / TBN) * ((g.m + TBM - 1) / TBM);
   const bool pool = s && s->queue_pool && tiles <= kPoolTiles;
-  int splits = tiled_splits(g.m, g.n, g.k, g.canonical,
-                            pool ? kPoolFloats : (s && s->partials) ? s->partial_floats : 0);
-  if (pool) splits = pool_splits(splits, tiles, TBM * TBN, kTileRounds * pool_max_splits(TBM / (256 / (TBN / 4))), steps);
   p.steps_per_split = (steps + splits - 1) / splits;
   p.partials = splits > 1 && !pool ? s->partials : nullptr;
   p.pool = pool;
@@ -3644,7 +3658,7 @@ hipError_t gemm(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* de
     return launch_panel(g, s, stream, deferred);
   }
   if (wvec && avec) {
-    const hipError_t e = g.w_int8 ? launch_row_tiles<TW_ROW8>(g, stream) : launch_row_tiles<TW_ROW16>(g, stream);
+    const hipError_t e = g.w_int8 ? launch_row_tiles<TW_ROW8>(g, s, stream) : launch_row_tiles<TW_ROW16>(g, s, stream);
     if (e != hipErrorNotSupported) return e;
   }
   // (fp16 rows of no whole 4-column groups, over columns that fill the chip by
