@@ -1,0 +1,57 @@
+"""Dispatch rules by their times: of two calls that share the work, or whose work
+differs by a known factor, neither may take far longer than the other.  Each
+bound lies between what a right choice and a wrong one measured on MI355X, at
+least a fifth away from the right one."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def torch():
+    import torch as t
+    return t
+
+
+def times(*calls):
+    """Best time in us of each call among 24 queued ones, the calls timed in turn."""
+    t = torch()
+    best = [float("inf")] * len(calls)
+    for call in calls:
+        call()
+    t.cuda.synchronize()
+    for _ in range(7):
+        for i, call in enumerate(calls):
+            start, end = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(24):
+                call()
+            end.record()
+            end.synchronize()
+            best[i] = min(best[i], start.elapsed_time(end) * 1e3 / 24)
+    return best
+
+
+def attention(ops, batch, heads, nq, nk, d, causal):
+    t = torch()
+    gen = t.Generator(device="cuda").manual_seed(batch)
+    q, k, v = (t.randn(batch, heads, n, d, generator=gen, device="cuda").half() for n in (nq, nk, nk))
+    off = [nk - nq] * batch
+    return lambda: ops.attention(q, k, v, query_offsets=off, causal=causal)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_few_attention_rows_use_every_xcd(ops, d):
+    """4 heads of 4096 queries against 8: half the work (28 and 58 us at 64 dims;
+    57 and 58 with whole rows on single XCDs)."""
+    print("[case] attention rows", d, flush=True)
+    half, whole = times(attention(ops, 1, 4, 4096, 4096, d, False), attention(ops, 1, 8, 4096, 4096, d, False))
+    assert half < 0.75 * whole, (half, whole)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_many_attention_rows_keep_their_l2_share(ops, causal):
+    """32 requests against 8 of the same shape: four times the work (295 and 85 us
+    without a mask; 555 and 101 with every row of an XCD in flight)."""
+    print("[case] attention batch", causal, flush=True)
+    small, large = times(attention(ops, 8, 25, 333, 1500, 128, causal), attention(ops, 32, 25, 333, 1500, 128, causal))
+    assert large < 4.6 * small, (small, large)

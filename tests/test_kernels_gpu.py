@@ -1130,6 +1130,8 @@ def test_non_default_stream_and_input_lifetime(ops):
 @pytest.mark.parametrize("batch,heads,nq,nk,d,causal", [
     (1, 1, 2, 2, 64, True), (1, 3, 65, 70, 128, True), (3, 3, 130, 130, 64, True),     # rows no multiple of 8
     (8, 25, 200, 256, 64, True), (5, 13, 129, 300, 128, False), (3, 33, 1000, 1000, 64, True),
+    (3, 5, 40, 90, 128, True), (4, 12, 330, 330, 64, True), (1, 4, 1100, 1100, 64, False),  # one tile; together; in turn
+    (15, 19, 330, 340, 128, True), (5, 13, 700, 720, 128, False), (1, 109, 400, 900, 64, False),  # groups and a rest
 ])
 def test_prefill_attention_every_row_and_tile(ops, batch, heads, nq, nk, d, causal):
     """Each (b, h) row and query tile is taken once, whatever the row count, with

@@ -47,6 +47,8 @@ __device__ __forceinline__ int written_queries(const AttnArgs& a, int q_valid) {
   return a.q_row_start ? q_valid : a.q_len;
 }
 
+constexpr int kRowsInTurn = 0, kRowsTogether = -1;
+
 struct AttnParams {
   AttnArgs a;
   float scale;
@@ -55,7 +57,10 @@ struct AttnParams {
                   // chunk's (m, l, unnormalized acc) in the queue's pool slot,
                   // merged by the row's last chunk to finish
   int chunks;     // split decode: key chunks per (b, h)
-  bool flat;      // prefill: one-dimensional grid, heaviest query tiles first
+  int group;      // prefill: rows an XCD walks together, heaviest query tiles
+                  // first, over a one-dimensional grid; kRowsTogether: all of
+                  // them, over (heads, batch, query tiles); kRowsInTurn: row
+                  // after row, over (query tiles, heads, batch)
 };
 
 template <bool VEC>
@@ -525,6 +530,9 @@ constexpr int kPrefillSplitTiles = 8;
 constexpr size_t kPrefillPoolFloats = size_t(kPrefillPoolTiles) * 2 * 256 * (64 / 16 * 4 + 2);  // acc, then (m, l)
 TIA_QUEUE_POOL_N(pf_pool, kPrefillSlots, kPrefillPoolFloats, kPrefillPoolTiles)
 
+// Query tile at place k of a row walked light and heavy in turn: 0, n-1, 1, n-2, ...
+__device__ __forceinline__ int light_heavy(int k, int n) { return (k & 1) ? n - 1 - (k >> 1) : (k >> 1); }
+
 template <int D, int KS, int QB = 1, bool SPLITKV = false>
 __global__ __launch_bounds__(256 * KS, prefill_waves_per_simd(D, KS, QB)) void prefill_mfma_kernel(AttnParams p) {
   static_assert(!SPLITKV || (D == 64 && QB == 1), "split prefill: 64-dim heads, one query block");
@@ -545,29 +553,45 @@ __global__ __launch_bounds__(256 * KS, prefill_waves_per_simd(D, KS, QB)) void p
   const int j = lane & 15, g = lane >> 4;
   // Workgroups go to the 8 XCDs round-robin by linear id.  Taken as is, the
   // grid (query tiles, heads, batch) would fetch the K and V of one (b, h) into
-  // eight L2s; each XCD gets whole (b, h) rows instead.
-  // A flat grid (p.flat) walks each XCD's rows by query tile, the last tiles
-  // (under the causal mask the heaviest) of every row first, so the workgroups
-  // that finish a launch are its lightest: B8 H25 1024^2 causal 71 -> 53 us
-  // against whole rows in turn, B4 H16 1024^2 D128 54 -> 41, B32 H12 512^2 42 -> 34.
-  // Its rows go to the XCDs one by one, so requests of unlike lengths spread
-  // over all of them: B2 H25 2000^2, lengths 1000 and 2000, 92 -> 67 us, B4 H16
-  // 333 x 700..1500 D128 49 -> 44 against contiguous rows per XCD.
-  // Otherwise (a grid too large to be flat) ids are regrouped into 8
-  // contiguous runs of whole rows, within a row the query tiles alternating
-  // light and heavy (0, n-1, 1, n-2, ...).
+  // eight L2s; each XCD gets whole (b, h) rows instead, one by one, so requests
+  // of unlike lengths spread over all of them (B2 H25 2000^2, lengths 1000 and
+  // 2000, 92 -> 67 us against contiguous rows per XCD).  The tiles of the
+  // rows % 8 that are left go to the XCDs in eight equal runs, light and heavy
+  // ones in turn: whole rows would leave XCDs idle (B1 H4 4096^2 without a mask
+  // 57 us, in runs 30).
+  // A group of rows is walked by query tile, the last tiles (under the causal
+  // mask the heaviest) of every row first, so the workgroups that finish a launch
+  // are its lightest (order_prefill has the sizes and figures).
+  // kRowsInTurn: ids are regrouped into 8 contiguous runs of whole rows, within a
+  // row the query tiles alternating light and heavy.
   // SPLITKV: an XCD's run of R ids (R even) holds half 0 of its R / 2 tiles
   // in its first R / 2 ids and half 1 of the same tiles, in reverse order, in
   // the rest, so the two workgroups a CU takes in turn (run positions c and
   // c + R / 2) pair a light tile's half with a heavy tile's.
   int b, h, q0, part = 0, tile_id = 0;
-  if (!SPLITKV && p.flat) {
-    const int nq = (a.q_len + BQ - 1) / BQ, rows = a.heads * a.batch, per = (rows + 7) >> 3;
-    const int c = int(blockIdx.x) >> 3, k = c / per, row = c % per * 8 + (int(blockIdx.x) & 7);
-    if (row >= rows) return;
+  if (!SPLITKV && p.group == kRowsTogether) {
+    h = int(blockIdx.x);
+    b = int(blockIdx.y);
+    q0 = int(gridDim.z - 1 - blockIdx.z) * BQ;
+  } else if (!SPLITKV && p.group != kRowsInTurn) {
+    const int nq = (a.q_len + BQ - 1) / BQ, rows = a.heads * a.batch;
+    const int per = rows >> 3, rest = rows & 7, run = (rest * nq + 7) >> 3;  // an XCD's whole rows, and its run of the rest
+    const int x = int(blockIdx.x) & 7, c = int(blockIdx.x) >> 3;
+    int k, row;
+    if (c < run) {
+      const int li = x * run + c;
+      if (li >= rest * nq) return;
+      k = light_heavy(li % nq, nq);
+      row = 8 * per + li / nq;
+    } else {
+      const int first = (c - run) / (p.group * nq) * p.group, at = c - run - first * nq;
+      const int size = min(p.group, per - first);
+      k = nq - 1 - at / size;
+      row = (first + at % size) * 8 + x;
+    }
     h = row % a.heads;
     b = row / a.heads;
-    q0 = (nq - 1 - k) * BQ;
+    q0 = k * BQ;
   } else {
     constexpr int PARTS = SPLITKV ? 2 : 1;
     const int nx = int(gridDim.x), nq = nx / PARTS, nh = int(gridDim.y);
@@ -592,7 +616,7 @@ __global__ __launch_bounds__(256 * KS, prefill_waves_per_simd(D, KS, QB)) void p
     const int k = li % nq, row = li / nq;
     h = row % nh;
     b = row / nh;
-    q0 = ((k & 1) ? nq - 1 - (k >> 1) : (k >> 1)) * BQ;
+    q0 = light_heavy(k, nq) * BQ;
   }
 
   const int q_valid = max(0, min(a.q_len, a.q_lengths[b]));
@@ -943,6 +967,39 @@ size_t max_lds_per_block() {
   return size_t(n);
 }
 
+// Order of a prefill launch (AttnParams::group) and its grid.  The workgroups an
+// XCD runs at once share the K and V they read through its L2 the more, the
+// fewer rows they come from; the more rows are walked together, the shorter a
+// causal launch's end, which runs light tiles instead of heavy ones.  us on MI355X,
+// all of an XCD's rows together / in groups / row after row:
+// * causal, 64 dims: together (B8 H25 1024^2, 25 rows per XCD, 47 / 49 / 60; B32
+//   H12 512^2 32 / 31 / 38); 128 dims, where K and V are twice as wide, in groups
+//   of 8 from 33 rows or 16 MB of them and 192 workgroups per XCD: B32 H12 512^2
+//   80 / 64 / 76, B32 H25 333 x 1500 497 / 276 / 270, B8 H25 333 x 1500 (25 rows)
+//   88 / 78 / 75, B32 H25 128^2 31.6 / 24.9 / 27.8, but B8 H25 1024^2 with lengths
+//   205..1024 65 / 68 / 68, B32 H12 128^2 14.2 / 15 / 15.3;
+// * no mask, where tiles weigh alike: in pairs, B32 H12 512^2 D128 125 / 91 / 92, B8
+//   H25 1024^2 D128 214 / 168 / 169; together while the L2 holds every row (B8 H12
+//   512^2 13.9 / 14.6 / 14.5);
+// * one tile per row: rows one by one, nothing to order; at most one workgroup per
+//   CU, or fewer rows than XCDs: in turn.
+int order_prefill(const AttnArgs& a, int tile, int threads, dim3& grid) {
+  const int64_t rows = int64_t(a.heads) * a.batch, nq = (a.q_len - 1) / tile + 1, per = rows / 8;
+  if (nq > 1 && (rows < 8 || rows * nq <= 256)) return kRowsInTurn;
+  const int64_t bytes = per * a.kv_len * a.head_dim * 4;  // K and V of an XCD's rows
+  const bool together = !a.causal          ? bytes <= 2500000
+                        : a.head_dim == 64 ? true
+                                           : per * nq < 192 || (per <= 32 && bytes <= 16000000);
+  if (nq == 1 || (together && rows % 8 == 0 && nq <= 65535)) {
+    grid = dim3(unsigned(a.heads), unsigned(a.batch), unsigned(nq));
+    return kRowsTogether;
+  }
+  const int64_t ids = 8 * (per * nq + (rows % 8 * nq + 7) / 8);
+  if (ids * threads >= int64_t(1) << 32) return kRowsInTurn;  // (the threads of one grid dimension)
+  grid = dim3(unsigned(ids));
+  return int(together ? per : a.causal ? 8 : 2);
+}
+
 // K and V rows (pitch D + 16), two buffers per key group; the key-group merge
 // reuses them.
 template <int D, int KS, int QB, bool SPLITKV = false>
@@ -953,11 +1010,7 @@ hipError_t launch_prefill(dim3 grid, AttnParams p, hipStream_t stream) {
       reinterpret_cast<const void*>(&prefill_mfma_kernel<D, KS, QB, SPLITKV>), hipFuncAttributeMaxDynamicSharedMemorySize,
       int(lds));
   if (attr != hipSuccess) return attr;
-  // (Rows rounded up to whole eights, one run per XCD; a launch takes fewer than
-  // 2^32 threads in one dimension.)
-  const int64_t flat = (int64_t(p.a.heads) * p.a.batch + 7) / 8 * 8 * ((p.a.q_len - 1) / (64 * QB) + 1);
-  p.flat = !SPLITKV && flat * 256 * KS < (int64_t(1) << 32);
-  if (p.flat) grid = dim3(unsigned(flat));
+  if (!SPLITKV) p.group = order_prefill(p.a, 64 * QB, 256 * KS, grid);
   hipLaunchKernelGGL((prefill_mfma_kernel<D, KS, QB, SPLITKV>), grid, dim3(256 * KS), lds, stream, p);
   return hipGetLastError();
 }
