@@ -974,22 +974,22 @@ size_t max_lds_per_block() {
 // all of an XCD's rows together / in groups / row after row:
 // * causal, 64 dims: together (B8 H25 1024^2, 25 rows per XCD, 47 / 49 / 60; B32
 //   H12 512^2 32 / 31 / 38); 128 dims, where K and V are twice as wide, in groups
-//   of 8 from 33 rows or 16 MB of them and 192 workgroups per XCD: B32 H12 512^2
-//   80 / 64 / 76, B32 H25 333 x 1500 497 / 276 / 270, B8 H25 333 x 1500 (25 rows)
-//   88 / 78 / 75, B32 H25 128^2 31.6 / 24.9 / 27.8, but B8 H25 1024^2 with lengths
-//   205..1024 65 / 68 / 68, B32 H12 128^2 14.2 / 15 / 15.3;
+//   of 8 from 33 rows of 192 workgroups per XCD, or 16 MB: B32 H12 512^2 80 / 64 /
+//   76, B32 H25 333 x 1500 497 / 276 / 270, B8 H25 333 x 1500 (25 rows) 88 / 78 /
+//   75, B32 H25 128^2 31.6 / 24.9 / 27.8, but B8 H25 1024^2 with lengths 205..1024
+//   65 / 68 / 68, B32 H12 128^2 14.2 / 15 / 15.3;
 // * no mask, where tiles weigh alike: in pairs, B32 H12 512^2 D128 125 / 91 / 92, B8
-//   H25 1024^2 D128 214 / 168 / 169; together while the L2 holds every row (B8 H12
-//   512^2 13.9 / 14.6 / 14.5);
+//   H25 1024^2 D128 214 / 168 / 169, B3 H25 333^2 D128 18.5 / 17.1 / 17.1; together
+//   while the L2 holds every row and none are left (B8 H12 512^2 13.9 / 14.6 / 14.5);
 // * one tile per row: rows one by one, nothing to order; at most one workgroup per
 //   CU, or fewer rows than XCDs: in turn.
 int order_prefill(const AttnArgs& a, int tile, int threads, dim3& grid) {
   const int64_t rows = int64_t(a.heads) * a.batch, nq = (a.q_len - 1) / tile + 1, per = rows / 8;
   if (nq > 1 && (rows < 8 || rows * nq <= 256)) return kRowsInTurn;
   const int64_t bytes = per * a.kv_len * a.head_dim * 4;  // K and V of an XCD's rows
-  const bool together = !a.causal          ? bytes <= 2500000
+  const bool together = !a.causal          ? rows % 8 == 0 && bytes <= 2500000
                         : a.head_dim == 64 ? true
-                                           : per * nq < 192 || (per <= 32 && bytes <= 16000000);
+                                           : bytes <= 16000000 && (per <= 32 || per * nq < 192);
   if (nq == 1 || (together && rows % 8 == 0 && nq <= 65535)) {
     grid = dim3(unsigned(a.heads), unsigned(a.batch), unsigned(nq));
     return kRowsTogether;
