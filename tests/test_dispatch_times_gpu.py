@@ -2,6 +2,8 @@
 differs by a known factor, neither may take far longer than the other.  Each
 bound lies between what a right choice and a wrong one measured on MI355X, at
 least a fifth away from the right one."""
+import itertools
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +57,31 @@ def test_many_attention_rows_keep_their_l2_share(ops, causal):
     print("[case] attention batch", causal, flush=True)
     small, large = times(attention(ops, 8, 25, 333, 1500, 128, causal), attention(ops, 32, 25, 333, 1500, 128, causal))
     assert large < 4.6 * small, (small, large)
+
+
+def linear(ops, kind, m, k, n, out="f16"):
+    """An int8 or fp16 linear over weights that rotate, as a model's layers."""
+    t = torch()
+    gen = t.Generator(device="cuda").manual_seed(m + k + n)
+    a = t.randn(m, k, generator=gen, device="cuda").half()
+    sets = max(1, min(24, (300 << 20) // (k * n)))
+    w = t.randint(-127, 128, (sets, k, n), generator=gen, device="cuda", dtype=t.int8)
+    if kind == "fp16":
+        w = w.half()
+    s = t.rand(n, generator=gen, device="cuda") * 1e-3
+    dtype = t.float32 if out == "f32" else t.float16
+    at = itertools.count()
+
+    def call():
+        held = w[next(at) % sets]
+        return ops.gemm_int8(a, held, s, output_dtype=dtype) if kind == "int8" else ops.gemm(a, held, output_dtype=dtype)
+    return call
+
+
+@pytest.mark.parametrize("kind,k", [("int8", 3072), ("fp16", 6400)])
+def test_few_columns_above_1024_rows_split_k(ops, kind, k):
+    """fp32 outputs take the kernel that splits K; fp16 ones of the same product
+    need not be slower (int8: 15 and 15 us; 42 and 15 as one chain over K)."""
+    print("[case] few columns", kind, k, flush=True)
+    half, single = times(linear(ops, kind, 1100, k, 64), linear(ops, kind, 1100, k, 64, out="f32"))
+    assert half < 1.6 * single, (half, single)

@@ -3493,24 +3493,43 @@ int tiled_plan(const GemmArgs& g, const Scratch* s) {
 //   25.8; below, 1024 x 768 x 768 12.1 / 9.8, 512 x 3072 x 768 36 / 14.8 (fp16 34 /
 //   17); the longest K keeps the row GEMM up to 144 tiles of 128 x 128
 //   (1024 x 6400 x 1600 87 / 83);
-// * above, the tiled kernel only where K is no multiple of 8: 1500 x 768 x 768
-//   12.1 / 16.4, 1500 x 3072 x 768 44 / 64;
+// * above, the tiled kernel where it has splits of K to run at once (weights from
+//   HBM): int8 1100 x 3072 x 64 41.7 / 14.8, 1100 x 6400 x 300 88 / 69, 1500 x 768
+//   x 300 14.9 / 13.2, unsplit 2000 x 768 x 300 15 / 18; fp16, which converts
+//   nothing, from three splits, or two at long K: 1100 x 3072 x 64 36 / 15, 1100
+//   x 6400 x 300 94 / 83, but 1500 x 768 x 300 11.9 / 13.2;
+// * above, at short K, where a chunk of 64 that is not full costs as much as a
+//   full one and filling the pipeline as much as the work: int8 1856 x 144 x 768
+//   7.7 / 6.8, 1136 x 96 x 1600 6.2 / 5.7, 1100 x 304 x 300 10.1 / 9.3, from 600 tiles
+//   of 64 x 64 on 2146 x 64 x 3576 7.7 / 10.9; with GELU, which a launch of few
+//   long-lived tiles does not overlap, 1364 x 72 x 2304 9.6 / 8.3, 5650 x 72 x 768
+//   11.9 / 10.3, 1310 x 144 x 2304 11.1 / 9.4; fp16 1288 x 160 x 768 7.2 / 6.4;
 // * fp32 outputs show the length of the sums that 16 bits hide, and here every
 //   one is a single chain over K: they stay with the kernels that cut K (the int8
 //   row GEMM up to kRowMaxM rows, the tiled kernel where it splits).  Distance
 //   from 64-bit sums, this kernel against them: 1024 x 768 x 3072 1.8e-7 / 8.7e-8
 //   (15.1 / 25.8 us), 1024 x 1600 x 6400 2.5e-7 / 1.1e-7.
 template <int TW>
+bool row_tiles_preferred(const GemmArgs& g, const Scratch* s) {
+  const int splits = tiled_plan(g, s);
+  if ((g.epi.kind == EPI_F32 || g.epi.kind == EPI_RAW_F32) && ((TW == TW_ROW8 && g.m <= kRowMaxM) || splits > 1))
+    return false;
+  if (g.m <= kRowMaxM)
+    return tiles_of(g.m, g.n, 128, 128) >= 144 || (tiles_of(g.m, g.n, 64, 128) >= 160 && g.k <= 4096);
+  const int64_t tiles = tiles_of(g.m, g.n, 64, 64);
+  const bool ragged = g.k % 64 != 0, gelu = g.epi.kind == EPI_GELU;
+  if constexpr (TW == TW_ROW16) return !(splits > 2 || (splits == 2 && g.k > 1600) || (tiles < 400 && ragged && g.k < 256));
+  if (splits > 1 || (tiles < 600 && g.k < (ragged ? 400 : gelu ? 200 : 176))) return false;
+  return !gelu || g.k >= 240 || (g.k >= 128 && tiles >= 800);
+}
+
+template <int TW>
 hipError_t launch_row_tiles(const GemmArgs& g, const Scratch* s, hipStream_t stream) {
   const int64_t ldw = g.ldw > 0 ? g.ldw : g.n;
-  if (g.k % 8 != 0 || g.lda > (1 << 22) || ldw > (1 << 24) || g.epi.kind == EPI_QKV || g.epi.p32 || g.m <= 32)
+  if (g.k % 8 != 0 || g.lda > (1 << 22) || ldw > (1 << 24) || g.epi.kind == EPI_QKV || g.epi.p32 || g.m <= 32 ||
+      !row_tiles_preferred<TW>(g, s))
     return hipErrorNotSupported;
-  if ((g.epi.kind == EPI_F32 || g.epi.kind == EPI_RAW_F32) &&
-      ((TW == TW_ROW8 && g.m <= kRowMaxM) || tiled_plan(g, s) > 1))
-    return hipErrorNotSupported;
-  const int64_t mid = tiles_of(g.m, g.n, 128, 128);
-  if (mid >= 144) return launch_tile<TW>(g, stream);
-  if (g.m <= kRowMaxM && (tiles_of(g.m, g.n, 64, 128) < 160 || g.k > 4096)) return hipErrorNotSupported;
+  if (tiles_of(g.m, g.n, 128, 128) >= 144) return launch_tile<TW>(g, stream);
   return TW == TW_ROW8 ? launch_tile_cfg<TW, 2, 2, 2, 4, 2, 2>(g, 0, g.m, stream)
                        : launch_tile_cfg<TW, 2, 1, 2, 4, 2, 2>(g, 0, g.m, stream);
 }
