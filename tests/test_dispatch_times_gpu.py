@@ -85,3 +85,12 @@ def test_few_columns_above_1024_rows_split_k(ops, kind, k):
     print("[case] few columns", kind, k, flush=True)
     half, single = times(linear(ops, kind, 1100, k, 64), linear(ops, kind, 1100, k, 64, out="f32"))
     assert half < 1.6 * single, (half, single)
+
+
+@pytest.mark.parametrize("m,k,n", [(866, 3072, 1600), (523, 2160, 2304)])
+def test_long_sums_over_few_tiles_cut_k(ops, m, k, n):
+    """fp32 outputs take the kernel that cuts K over waves; fp16 ones of the same
+    product need not be slower (35 and 37 us; 53 as one chain over K)."""
+    print("[case] long sums", m, k, n, flush=True)
+    half, single = times(linear(ops, "int8", m, k, n), linear(ops, "int8", m, k, n, out="f32"))
+    assert half < 1.2 * single, (half, single)
