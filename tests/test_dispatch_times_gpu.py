@@ -94,3 +94,11 @@ def test_long_sums_over_few_tiles_cut_k(ops, m, k, n):
     print("[case] long sums", m, k, n, flush=True)
     half, single = times(linear(ops, "int8", m, k, n), linear(ops, "int8", m, k, n, out="f32"))
     assert half < 1.2 * single, (half, single)
+
+
+def test_odd_wide_rows_at_short_k(ops):
+    """int8 rows of any alignment at short K are no slower than fp16 ones of twice
+    the bytes (105 and 97 us; 241 with each weight converted once per 32 rows)."""
+    print("[case] odd wide rows", flush=True)
+    int8, fp16 = times(linear(ops, "int8", 1024, 64, 50257), linear(ops, "fp16", 1024, 64, 50257))
+    assert int8 < 1.5 * fp16, (int8, fp16)

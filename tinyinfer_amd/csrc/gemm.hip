@@ -2354,6 +2354,9 @@ hipError_t launch_rowgemv(const GemmArgs& g, hipStream_t stream) {
 // of 16-row blocks has more than 8 steps; S steps a round, rounds repeated
 // over longer splits.
 constexpr int kRowMaxM = 1024;
+// 16-row blocks of a workgroup.  (A 16-row block would read the weights once per
+// block; once the column tiles alone fill the chip, 32 rows share them.)
+int rowgemm_blocks16(int m, int ntile) { return m <= 64 && ntile < kRowTargetBlocks ? 1 : 2; }
 template <bool INT8, bool WVEC, int MT, int W, int S>
 hipError_t launch_rowgemm_ws(const SkinnyParams& p, hipStream_t stream) {
   hipLaunchKernelGGL((rowgemm_kernel<INT8, WVEC, MT, W, S>), dim3(unsigned(p.ntile * p.rblocks * p.splits)), dim3(W * 64), 0,
@@ -2368,9 +2371,7 @@ hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   p.ldw = g.ldw > 0 ? g.ldw : g.n;
   p.ntile = (g.n + 63) / 64;
   p.steps = (g.k + 31) / 32;
-  // (A 16-row block would read the weights once per block; once the column
-  // tiles alone fill the chip, 32 rows share them.)
-  const int mt = g.m <= 64 && p.ntile < kRowTargetBlocks ? 1 : 2;
+  const int mt = rowgemm_blocks16(g.m, p.ntile);
   p.rblocks = (g.m + 16 * mt - 1) / (16 * mt);
   const int64_t units = int64_t(p.ntile) * p.rblocks;
   int splits = int(std::clamp<int64_t>((kRowTargetBlocks + units / 2) / units, 1, rowgemm_max_splits(mt, 8)));
@@ -3532,6 +3533,35 @@ bool row_tiles_preferred(const GemmArgs& g, const Scratch* s) {
   return !(tiles < 600 && g.k < (ragged ? 400 : 200)) && (g.k >= 240 || (g.k >= 128 && tiles >= 800));
 }
 
+// Whether the row GEMM takes M in 33 .. kRowMaxM, or the tiled kernel (us, row GEMM
+// against tiled; a unit is the row GEMM's 32 rows x 64 columns).
+// * Whole aligned 4-column groups (wvec): int8 always; fp16 from where a tile's few
+//   K steps no longer run out before the row GEMM has started, later where its
+//   units are split (up to 128) or many: 393 x 80 x 1600 5.7 / 5.0, 300 x 144 x 1600
+//   5.3 / 6.4, 69 x 88 x 96 5.7 / 4.1, 210 x 168 x 332 6.4 / 7.0, 906 x 232 x 1192 9.5 /
+//   8.9 (551 units), 491 x 768 x 2432 20.0 / 22.7.
+// * Rows of any alignment, short K: only unsplit units that fit the chip about
+//   twice, 64 x 64 x 2305 5.0 / 6.5, 128 x 64 x 6399 5.9 / 6.5, but 65 x 64 x 301
+//   6.4 / 4.8, 1024 x 64 x 6399 32 / 18, 1024 x 64 x 50257 241 / 105.
+// * Rows of any alignment, more tiles than half a round (five per CU) of the tiled
+//   kernel: by their costs in us, the row GEMM's per unit and per unit and step,
+//   the tiled kernel's per round and per tile of a step.  fp16: 512 x 768 x 6399
+//   55 / 52, 768 x 1600 x 6399 119 / 108, 1024 x 1600 x 6399 152 / 185 (a second
+//   round), 99 x 1704 x 25001 86 / 118; int8: 465 x 288 x 50257 142 / 133, 512 x 768 x
+//   50257 247 / 314.
+bool row_gemm_preferred(const GemmArgs& g, bool wvec) {
+  const int ntile = (g.n + 63) / 64, rows = 16 * rowgemm_blocks16(g.m, ntile), steps = (g.k + 31) / 32;
+  const int64_t units = int64_t(ntile) * ((g.m + rows - 1) / rows), tiles = tiles_of(g.m, g.n, TBM, TBN);
+  if (wvec) return g.w_int8 || g.k > (units > 512 ? 255 : units > 128 ? 128 : 144);
+  if (g.k <= 160 && (units > 512 || (units <= 128 && g.k <= 96))) return false;
+  const int64_t round = int64_t(5) * device_cus();
+  if (2 * tiles <= round) return true;
+  const double row = double(units) * (g.w_int8 ? 0.0066 + 0.00055 * steps : 0.014 + 0.00067 * steps) + 5;
+  const double tiled = steps * ((g.w_int8 ? 2.3 : 1.6) * double((tiles + round - 1) / round) +
+                                (g.w_int8 ? 0.0006 : 0.0004) * double(tiles)) + 5;
+  return row <= tiled;
+}
+
 template <int TW>
 hipError_t launch_row_tiles(const GemmArgs& g, const Scratch* s, hipStream_t stream) {
   const int64_t ldw = g.ldw > 0 ? g.ldw : g.n;
@@ -3689,10 +3719,8 @@ hipError_t gemm(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* de
     const hipError_t e = g.w_int8 ? launch_row_tiles<TW_ROW8>(g, s, stream) : launch_row_tiles<TW_ROW16>(g, s, stream);
     if (e != hipErrorNotSupported) return e;
   }
-  // (fp16 rows of no whole 4-column groups, over columns that fill the chip by
-  // themselves: the tiled kernel from 33 rows, M = 64 768 x 50257 51 against 55 us.)
-  const bool tiled_fp16 = !g.w_int8 && !wvec && g.m > 32 && g.n >= 64 * kRowTargetBlocks;
-  if (g.m <= kRowMaxM && g.n >= 4 && avec && g.k % 8 == 0 && s && s->queue_pool && !deferred && !tiled_fp16) {
+  if (g.m <= kRowMaxM && g.n >= 4 && avec && g.k % 8 == 0 && s && s->queue_pool && !deferred &&
+      (g.m <= 32 || row_gemm_preferred(g, wvec))) {
     const hipError_t e = g.w_int8 ? (wvec ? launch_row<true, true>(g, stream) : launch_row<true, false>(g, stream))
                                   : (wvec ? launch_row<false, true>(g, stream) : launch_row<false, false>(g, stream));
     if (e != hipErrorNotSupported) return e;
