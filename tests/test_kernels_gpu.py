@@ -642,6 +642,31 @@ def test_row_major_any_alignment(ops, m, n, k, int8):
         assert bool(((out.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("kind,m,n,k,most", [
+    ("fp16", 4, 3072, 2784, 6.9e-8), ("fp16", 4, 1600, 5648, 8.4e-8), ("fp16", 27, 5255, 3072, 8e-8),
+    ("fp16", 31, 4800, 6400, 1.12e-7), ("int8", 12, 5170, 1600, 4.7e-8), ("int8", 27, 5255, 3072, 6.1e-8),
+])
+def test_few_rows_sum_in_short_chains(ops, kind, m, n, k, most):
+    """fp32 outputs at few rows: relative distance (2-norm) from 64-bit sums.  `most`
+    is what the skinny kernel, which these row kernels stand in for, measured (K
+    over four waves and up to 43 splits) and 3 % for other values; one chain over
+    the waves and one over the splits measured 1.1 to 1.2 times that."""
+    t = torch()
+    say("short chains", kind, m, n, k)
+    gen = t.Generator(device="cuda").manual_seed(m + n + k)
+    a = t.randn(m, k, generator=gen, device="cuda").half()
+    bias = t.randn(n, generator=gen, device="cuda").half()
+    if kind == "int8":
+        q = t.randint(-127, 127, (k, n), generator=gen, device="cuda", dtype=t.int8)
+        s = t.rand(n, generator=gen, device="cuda") * 1e-4 + 1e-4
+        w, out = (q.float() * s).half(), ops.gemm_int8(a, q, s, bias=bias, output_dtype=t.float32)
+    else:
+        w = (t.randn(k, n, generator=gen, device="cuda") * 0.02).half()
+        out = ops.gemm(a, w, bias=bias, output_dtype=t.float32)
+    ref = a.double() @ w.double() + bias.double()
+    assert float((out.double() - ref).norm() / ref.norm()) <= most
+
+
 @pytest.mark.parametrize("m,n,k", [(1100, 2050, 96), (3601, 3841, 160), (5000, 3844, 32), (1100, 2050, 64)])
 def test_record_large_tiles(ops, m, n, k):
     """fp16 records: the value of every tile choice, and the bits of the

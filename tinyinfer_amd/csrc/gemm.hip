@@ -217,6 +217,17 @@ __device__ __forceinline__ int xcd_run_id(int id, int n) {
   return x * (n >> 3) + min(x, n & 7) + (id >> 3);
 }
 
+// Sum of x[0 .. N) by pairs, then pairs of pairs, ...: N fp32 terms in log2 N
+// roundings each (one after the other: up to N - 1).
+template <int N, typename T>
+__device__ __forceinline__ T pairwise_sum(T (&x)[N]) {
+#pragma unroll
+  for (int d = 1; d < N; d *= 2)
+#pragma unroll
+    for (int i = 0; i + d < N; i += 2 * d) x[i] += x[i + d];
+  return x[0];
+}
+
 struct SkinnyParams {
   const uint16_t* a;
   int64_t lda;
@@ -598,10 +609,10 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
     for (int v = 0; v < 4; ++v) red[wave][4 * g + v][4 * j + c] = acc[c][v];
   __syncthreads();
   auto wave_sum = [&](int row, int cc) {
-    float s = red[0][row][cc];
+    float x[W];
 #pragma unroll
-    for (int w = 1; w < W; ++w) s += red[w][row][cc];
-    return s;
+    for (int w = 0; w < W; ++w) x[w] = red[w][row][cc];
+    return pairwise_sum(x);
   };
   if (p.splits == 1) {
     for (int e = threadIdx.x; e < p.m * 64; e += W * 64) {
@@ -619,12 +630,8 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
     float v[kRowSplits];
 #pragma unroll
     for (int u = 0; u < kRowSplits; ++u) v[u] = u < p.splits ? ld_agent(parts + u * 1024 + e) : 0.f;
-    float s = v[0];
-#pragma unroll
-    for (int u = 1; u < kRowSplits; ++u)
-      if (u < p.splits) s += v[u];
     const int n = n0 + (e & 63);
-    if (n < p.n) apply_epilogue(p.epi, e >> 6, n, s);
+    if (n < p.n) apply_epilogue(p.epi, e >> 6, n, pairwise_sum(v));
   }
   depart(slot.ctr + tile * kCounterStride);
 }
@@ -649,6 +656,10 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   constexpr int R = 16 * MT, NT = W * 64;
   constexpr int OUT4 = (R * 16 + NT - 1) / NT;  // float4 outputs of a finishing thread
   constexpr int SMAX = kPoolLoads / OUT4;       // splits its one round of loads covers
+  // Sums of a wave: the longest K over 16 rows in two chains, as short as the
+  // skinny kernel's (int8 in aligned groups, 48 x 1600 x 6400 14.7 -> 16.4 us with a
+  // second chain, keeps one).
+  constexpr int AC = MT == 1 && S == 4 && !(INT8 && WVEC) ? 2 : 1;
   __shared__ float red[W][R][65];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 15, g = lane >> 4;
@@ -664,11 +675,13 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   float sc[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) sc[c] = INT8 && col + c < p.n ? p.scales[col + c] : 0.f;
-  float4_t acc[MT][4];
+  float4_t acc[AC][MT][4];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int i = 0; i < AC; ++i)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[t][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[i][t][c] = float4_t{0.f, 0.f, 0.f, 0.f};
   for (int base = s0 + wave; base < s1; base += W * S) {
     WFrag<INT8> f[S];
     half8_t a[S][MT];
@@ -689,7 +702,8 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
         for (int c = 0; c < 4; ++c) {
           const half8_t b = bfrag<INT8>(f[i], c, sc[c]);
 #pragma unroll
-          for (int t = 0; t < MT; ++t) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][t], b, acc[t][c], 0, 0, 0);
+          for (int t = 0; t < MT; ++t)
+            acc[i % AC][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][t], b, acc[i % AC][t][c], 0, 0, 0);
         }
       }
     }
@@ -700,7 +714,8 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) red[wave][16 * t + 4 * g + v][4 * j + c] = acc[t][c][v];
+      for (int v = 0; v < 4; ++v)
+        red[wave][16 * t + 4 * g + v][4 * j + c] = AC == 2 ? acc[0][t][c][v] + acc[AC - 1][t][c][v] : acc[0][t][c][v];
   __syncthreads();
   // float4 output q of the unit: row q / 16, columns 4 (q % 16) .. + 3.
   const int tid = int(threadIdx.x), nq = rows * 16;
@@ -709,10 +724,10 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
     f32x4_t v;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      float x = red[0][r][c0 + c];
+      float x[W];
 #pragma unroll
-      for (int w = 1; w < W; ++w) x += red[w][r][c0 + c];
-      v[c] = x;
+      for (int w = 0; w < W; ++w) x[w] = red[w][r][c0 + c];
+      v[c] = pairwise_sum(x);
     }
     return v;
   };
@@ -746,11 +761,7 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   for (int o = 0; o < OUT4; ++o) {
     const int q = tid + o * NT;
     if (q >= nq) continue;
-    f32x4_t sum = v[o][0];
-#pragma unroll
-    for (int u = 1; u < SMAX; ++u)
-      if (u < p.splits) sum += v[o][u];
-    epilogue4(q, sum);
+    epilogue4(q, pairwise_sum(v[o]));
   }
 }
 // Most splits of a rowgemm_kernel<MT, W, S> plan.
