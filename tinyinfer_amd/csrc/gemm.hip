@@ -237,6 +237,7 @@ struct SkinnyParams {
   int64_t ldw;         // row stride of W in elements (>= n)
   int ntile;           // ceil(N / 64)
   int rblocks;         // row blocks (rowgemm_kernel)
+  bool rows_first;     // workgroup order: row blocks of a tile first, or tiles of a row block
   int steps;           // ceil(K / 32)
   int steps_per_block; // K steps owned by one workgroup (its waves take every 4th)
   int splits;
@@ -663,12 +664,15 @@ __global__ __launch_bounds__(W * 64) void rowgemm_kernel(SkinnyParams p) {
   __shared__ float red[W][R][65];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 15, g = lane >> 4;
-  // Consecutive ids per XCD (blocks go round-robin over the 8 XCDs), column
-  // tile fastest: the two tiles that share a 128-byte weight line, and the
-  // tiles that share a row block's A rows, are read through one L2.
+  // Consecutive ids per XCD (blocks go round-robin over the 8 XCDs).  Column tile
+  // fastest, the tiles that share a row block's A rows are read through one L2;
+  // row block fastest, the row blocks that share a tile's weights, which the
+  // launch chooses where the weights outweigh A: M = 144, 3072->3304 27.1 -> 23 us,
+  // M = 216, 4280->6400 48.9 -> 44.3, M = 354, 688->2016 8.95 -> 8.57.
   const int logical = xcd_run_id(int(blockIdx.x), int(gridDim.x));
-  const int tile = logical % p.ntile, rest = logical / p.ntile;
-  const int rb = rest % p.rblocks, split = rest / p.rblocks;
+  const int inner = p.rows_first ? p.rblocks : p.ntile, unit_id = logical % (p.ntile * p.rblocks);
+  const int split = logical / (p.ntile * p.rblocks), in = unit_id % inner, out = unit_id / inner;
+  const int tile = p.rows_first ? out : in, rb = p.rows_first ? in : out;
   const int m0 = rb * R, rows = min(R, p.m - m0);
   const int s0 = split * p.steps_per_block, s1 = min(p.steps, s0 + p.steps_per_block);
   const int n0 = tile * 64, col = n0 + 4 * j;
@@ -2384,6 +2388,7 @@ hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   p.steps = (g.k + 31) / 32;
   const int mt = rowgemm_blocks16(g.m, p.ntile);
   p.rblocks = (g.m + 16 * mt - 1) / (16 * mt);
+  p.rows_first = int64_t(g.n) * (INT8 ? 1 : 2) > int64_t(2) * g.m;
   const int64_t units = int64_t(p.ntile) * p.rblocks;
   int splits = int(std::clamp<int64_t>((kRowTargetBlocks + units / 2) / units, 1, rowgemm_max_splits(mt, 8)));
   while (splits > 1 && units * splits * 16 * mt * 64 > int64_t(kPoolFloats)) --splits;
