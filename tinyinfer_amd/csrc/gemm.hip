@@ -3507,10 +3507,11 @@ int tiled_plan(const GemmArgs& g, const Scratch* s) {
 // split K over few tiles (us, this kernel against them):
 // * int8 up to kRowMaxM rows (the row GEMM): the tiles take about as long for 150
 //   of them (64 x 128) as for 512, K / 64 chunks of 1 us, the row GEMM what its
-//   M N K takes.  They meet at 140 + K / 12 tiles, at most 300 (weights from HBM,
-//   bias): 512 x 768 x 3072 (192 tiles) 17.9 / 16.6, 768 x 768 x 3072 20 / 22,
-//   866 x 3072 x 1600 53 / 35, 1000 x 1600 x 1600 30 / 27, 523 x 2160 x 2304 41 / 25,
-//   512 x 1600 x 4800 (304) 35 / 37, 590 x 4800 x 6400 87 / 125;
+//   M N K takes.  They meet at 140 + K / 12 tiles, at most 300, and at 300 where few
+//   rows share each weight from HBM: bias, 512 x 768 x 3072 (192 tiles) 17.9 /
+//   16.6, 768 x 768 x 3072 20 / 22, 866 x 3072 x 1600 53 / 35, 1000 x 1600 x 1600 30 /
+//   27, 523 x 2160 x 2304 41 / 25, 512 x 1600 x 4800 (304) 35 / 37, 590 x 4800 x 6400
+//   87 / 125, 208 x 584 x 6400 17.2 / 13.6, 283 x 928 x 6400 (250) 24.7 / 20;
 // * fp16 up to kRowMaxM rows (the row GEMM, which loads twice the bytes): from
 //   160 such tiles, 1024 x 768 x 3072 18 / 24; the longest K keeps the row GEMM up
 //   to 144 tiles of 128 x 128;
@@ -3524,8 +3525,9 @@ int tiled_plan(const GemmArgs& g, const Scratch* s) {
 //   7.7 / 6.8, 1136 x 96 x 1600 6.2 / 5.7, 2200 x 64 x 172 4.1 / 3.9, but 1500 x 304 x
 //   768 9.2 / 9.6, and from 600 tiles of 64 x 64 on 2146 x 64 x 3576 7.7 / 10.9; with
 //   GELU, which a launch of few long-lived tiles does not overlap, 1100 x 304 x 300
-//   10.1 / 9.3, 1364 x 72 x 2304 9.6 / 8.3, 5650 x 72 x 768 11.9 / 10.3, 1310 x 144 x
-//   2304 11.1 / 9.4; fp16 1288 x 160 x 768 7.2 / 6.4;
+//   10.1 / 9.3, 1364 x 72 x 2304 9.6 / 8.3, 5650 x 72 x 768 11.9 / 10.3, 5000 x 144 x
+//   1600 21 / 18; fp16 (and up to kRowMaxM rows) 1288 x 160 x 768 7.2 / 6.4, 512 x 144
+//   x 3072 7.7 / 7.1;
 // * fp32 outputs show the length of the sums that 16 bits hide, and here every
 //   one is a single chain over K: they stay with the kernels that cut K (the int8
 //   row GEMM up to kRowMaxM rows, the tiled kernel where it splits).  Distance
@@ -3538,15 +3540,17 @@ bool row_tiles_preferred(const GemmArgs& g, const Scratch* s) {
     return false;
   if (g.m <= kRowMaxM) {
     const int64_t wide = tiles_of(g.m, g.n, 64, 128);
-    if (TW == TW_ROW8) return wide >= std::min(140 + g.k / 12, 300);
-    return tiles_of(g.m, g.n, 128, 128) >= 144 || (wide >= 160 && g.k <= 4096);
+    if (TW == TW_ROW8) return wide >= (g.m < 400 && g.k >= 400 ? 300 : std::min(140 + g.k / 12, 300));
+    if (tiles_of(g.m, g.n, 128, 128) < 144 && (wide < 160 || g.k > 4096)) return false;
   }
   const int64_t tiles = tiles_of(g.m, g.n, 64, 64);
   const bool ragged = g.k % 64 != 0, gelu = g.epi.kind == EPI_GELU;
-  if constexpr (TW == TW_ROW16) return !(splits > 2 || (splits == 2 && g.k > 1600) || (tiles < 400 && ragged && g.k < 256));
+  if (TW == TW_ROW16 && tiles < 500 && ragged && g.k < 256) return false;
+  if (g.m <= kRowMaxM) return true;
+  if constexpr (TW == TW_ROW16) return splits < 2 || (splits == 2 && g.k <= 1600);
   if (splits > 1) return false;
   if (!gelu) return !(ragged ? tiles < 600 && g.k < 232 : tiles < 300 && g.k < 176);
-  return !(tiles < 600 && g.k < (ragged ? 400 : 200)) && (g.k >= 240 || (g.k >= 128 && tiles >= 800));
+  return !(tiles < 600 && g.k < (ragged ? 400 : 200)) && (g.k >= 240 || (g.k >= 176 && tiles >= 800));
 }
 
 // Whether the row GEMM takes M in 33 .. kRowMaxM, or the tiled kernel (us, row GEMM
