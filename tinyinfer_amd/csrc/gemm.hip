@@ -3455,9 +3455,12 @@ int64_t tiles_of(int m, int n, int bm, int bn) {
 // full (int8: the conversions are shared by twice the columns per barrier;
 // M = 2048, 768->3072 19.7 against 21.2 us as 128 x 128), else 128 x 128, two
 // workgroups per CU.
+// Records at short K take no 256 x 256 tiles: their epilogue, eight passes over
+// LDS with one workgroup per CU, runs beside nothing (M = 8192, 768->3072 with GELU
+// 73 us with them, 58 without; M = 8192, 1600->1600 56 against 58).
 template <int TW>
 hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
-  const int big = tile_big_rows(g.m, g.n);
+  const int big = TW == TW_REC16 && g.k < 1024 ? 0 : tile_big_rows(g.m, g.n);
   if (big > 0) {
     const hipError_t e = launch_tile_cfg<TW, 2, 4, 8, 4, 8, 2>(g, 0, std::min(big, g.m), stream);
     if (e != hipSuccess || big >= g.m) return e;
@@ -3598,17 +3601,20 @@ hipError_t launch_row_tiles(const GemmArgs& g, const Scratch* s, hipStream_t str
 // * the large tiles once they hold >= 144 of 128 x 128: M = 1280 768->3072
 //   13.9 us (int8 panels 19.2), 768->2304 13.0 (15.2), M = 512 1600->4800 20.5
 //   (25.9), M = 2560 1600->1600 26 (64 x 64 tiles 36); below, M = 1280 768->768
-//   11.7 (64 x 64 tiles 7.7);
+//   11.7 (64 x 64 tiles 7.7); at short K, where filling their pipeline costs as much
+//   as the work, from 520 - 5 K / 4: M = 1280 64->4000 (320) 12.2 (64 x 64 tiles
+//   10.3), M = 1500 128->3072 (288) 12.6 (11.2), M = 1024 256->3072 (192) 10.5 (9.4), but
+//   M = 2048 64->4000 (512) 12.9 (13.1), M = 1280 256->3072 (240) 10.8 (11.9);
 // * below that, 64 x 64 tiles on 8 waves (each 32 x 16) for M >= 2048 at
 //   K < 1536: M = 2048 768->768; the int8 panels elsewhere;
 // * at K >= 1536 the 64 x 64 tiles keep a 4-stage ring (two chunks of 32 in
 //   flight): M = 1024 3072->768 25.3 us against 31.5 with 3 stages, which time
 //   the same or better at K = 768 (6 stages: slower everywhere).
-bool f16_gemm_large(int m, int n) { return tiles_of(m, n, 128, 128) >= 144; }
-bool f16_gemm_preferred(int m, int n, int k) { return f16_gemm_large(m, n) || (m >= 2048 && k < 1536); }
+bool f16_gemm_large(int m, int n, int k) { return tiles_of(m, n, 128, 128) >= std::max(144, 520 - 5 * std::min(k, 512) / 4); }
+bool f16_gemm_preferred(int m, int n, int k) { return f16_gemm_large(m, n, k) || (m >= 2048 && k < 1536); }
 
 hipError_t launch_f16(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* deferred) {
-  if (f16_gemm_large(g.m, g.n) && g.lda <= (1 << 22)) return launch_tile<TW_REC16>(g, stream);
+  if (f16_gemm_large(g.m, g.n, g.k) && g.lda <= (1 << 22)) return launch_tile<TW_REC16>(g, stream);
   if (g.k >= 1536) return launch_f16_cfg<2, 4, 2, 1, 4, 1, 3>(g, s, stream, deferred);
   return launch_f16_cfg<2, 4, 2, 1, 3, 1, 3>(g, s, stream, deferred);
 }
