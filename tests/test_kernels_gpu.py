@@ -704,6 +704,8 @@ def test_legacy_fp32_gemm(ops):
     (768, 768, 40), (1000, 1001, 33), (1089, 1024, 97),     # 64 x 64 tiles, with and without 16-byte rows
     (1100, 1028, 68), (1600, 1284, 4),                      # 32 x 64 tiles
     (2048, 2048, 31), (2049, 2050, 65),                     # 128 x 128 tiles
+    (1, 1000, 16), (65, 129, 15), (1030, 1, 1),             # one step of 64 x 64 tiles
+    (700, 700, 17), (1600, 1284, 20), (2048, 2049, 17),     # ... and the shortest K of the others
 ])
 def test_legacy_fp32_gemm_tiles(ops, m, n, k):
     """Each tile choice at ragged edges, against 64-bit sums.  A k-term fp32 sum

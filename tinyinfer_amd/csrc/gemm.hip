@@ -3666,18 +3666,22 @@ void launch_f32_cfg(const float* a, const float* b, float* c, int m, int n, int 
 
 // Tile by the number of workgroups it leaves (M x K x N, us; before: one
 // 64 x 64 tile of scalar fmas per workgroup for every shape):
+// * 64 x 64 up to K = 16, one step of one wave, where the others of a K group would
+//   only meet: 16 x 1 x 1024 2.6 against 3.5 as 32 x 32 (before 3.05), 2048 x 16 x 2048
+//   7.4 against 8.7 as 128 x 128 (10.0);
 // * 128 x 128 from one full round of them: 2048^3 138 (124 TF/s; before 351);
 //   with too few, half the CUs idle (1024^3: 71);
 // * 32 x 32, eight waves sharing K, up to one round: 512 x 2048 x 512 20
 //   against 44 as 64 x 64 tiles (before 300), 300 x 1500 x 200 15 against 33;
 // * 32 x 32, four waves, while 64 x 64 tiles would fill less than half the CUs;
-// * 64 x 64 up to one round of them: 1024^3 25 (85 TF/s; before 163);
+// * 64 x 64 up to one round of them: 1024^3 23.8 (90 TF/s; before 163);
 // * 32 x 64, K over four waves, above that, where the last round of larger
 //   tiles would be thin: 2048 x 2048 x 640 64 against 78, 1536^3 80 against 87.
 //   Rows that allow no 16-byte loads keep 64 x 64 (1000 x 1003 x 1001: 35
 //   against 47): their loads cost more per tile.
 void launch_f32_mfma(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t stream) {
   auto tiles = [&](int64_t bm, int64_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); };
+  if (k <= 16 && n <= (1 << 28)) return launch_f32_cfg<64, 64, 4, 2, 1, 32>(a, b, c, m, n, k, stream);
   if (tiles(128, 128) >= 256) return launch_f32_cfg<128, 128, 2, 2, 2, 32>(a, b, c, m, n, k, stream);
   if (tiles(32, 32) <= 256) return launch_f32_cfg<32, 32, 1, 1, 8, 128>(a, b, c, m, n, k, stream);
   if (tiles(64, 64) < 128) return launch_f32_cfg<32, 32, 1, 1, 4, 64>(a, b, c, m, n, k, stream);
