@@ -21,6 +21,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lds_limit.hpp"
 #include "queue_scratch.hpp"
 
 namespace tia {
@@ -1006,10 +1007,9 @@ template <int D, int KS, int QB, bool SPLITKV = false>
 hipError_t launch_prefill(dim3 grid, AttnParams p, hipStream_t stream) {
   constexpr size_t lds = size_t(KS) * 2 * 2 * 64 * (D + 16) * 2;
   static_assert(KS == 1 || size_t(KS - 1) * 256 * (D / 16 * 4 + 2) * QB * 4 <= lds, "merge fits the tile buffers");
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&prefill_mfma_kernel<D, KS, QB, SPLITKV>), hipFuncAttributeMaxDynamicSharedMemorySize,
-      int(lds));
-  if (attr != hipSuccess) return attr;
+  static LdsLimit limit;
+  const hipError_t e = limit.raise(reinterpret_cast<const void*>(&prefill_mfma_kernel<D, KS, QB, SPLITKV>), int(lds));
+  if (e != hipSuccess) return e;
   if (!SPLITKV) p.group = order_prefill(p.a, 64 * QB, 256 * KS, grid);
   hipLaunchKernelGGL((prefill_mfma_kernel<D, KS, QB, SPLITKV>), grid, dim3(256 * KS), lds, stream, p);
   return hipGetLastError();

@@ -47,6 +47,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lds_limit.hpp"
 #include "queue_scratch.hpp"
 
 namespace tia {
@@ -2734,13 +2735,11 @@ hipError_t launch_panel_cfg(const GemmArgs& g, const Scratch* s, hipStream_t str
   constexpr int BM = WM * MT * 16, BN = WN * R * 16;
   constexpr int NL = (BM / 16) * 2 + BN / 16;
   constexpr size_t kLds = size_t(S) * NL * 1024 + BN * 4;
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&panel_gemm_kernel<WM, WN, MT, R, S>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
-  static hipError_t attr_pool = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&panel_gemm_kernel<WM, WN, MT, R, S, true>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
-  if (attr != hipSuccess) return attr;
-  if (attr_pool != hipSuccess) return attr_pool;
+  static LdsLimit limit, limit_pool;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(&panel_gemm_kernel<WM, WN, MT, R, S>), int(kLds));
+  if (e == hipSuccess)
+    e = limit_pool.raise(reinterpret_cast<const void*>(&panel_gemm_kernel<WM, WN, MT, R, S, true>), int(kLds));
+  if (e != hipSuccess) return e;
   PanelParams p{};
   p.a = g.a; p.lda = g.lda; p.w = static_cast<const u32x4_t*>(g.w_packed); p.scales = g.scales;
   p.m = g.m; p.n = g.n; p.k = g.k; p.epi = g.epi;
@@ -2969,14 +2968,11 @@ hipError_t launch_f16_cfg(const GemmArgs& g, const Scratch* s, hipStream_t strea
   constexpr int BM = WM * MT * 16, BN = WN * R * 16;
   constexpr int NL = BM / 16 + BN / 16;
   constexpr size_t kLds = std::max(size_t(S) * NL * 1024, size_t(BM / EP) * tile_pitch(BN) * 4);
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
-  if (attr != hipSuccess) return attr;
-  static hipError_t attr_pool =
-      EP == 1 ? hipFuncSetAttribute(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC, EP == 1>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds))
-              : hipSuccess;
-  if (attr_pool != hipSuccess) return attr_pool;
+  static LdsLimit limit, limit_pool;
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC>), int(kLds));
+  if (e == hipSuccess && EP == 1)
+    e = limit_pool.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC, EP == 1>), int(kLds));
+  if (e != hipSuccess) return e;
   F16GemmParams p{};
   p.a = g.a; p.lda = g.lda; p.w = static_cast<const u32x4_t*>(g.w_f16p);
   p.m = g.m; p.n = g.n; p.k = g.k; p.epi = g.epi;
@@ -3405,9 +3401,9 @@ hipError_t launch_tile_cfg(const GemmArgs& g, int m_begin, int m_end, hipStream_
   constexpr bool REC = TW == TW_REC16;
   constexpr size_t kLds = tile_lds_ring<TW, BM, BN, EP>() + (REC ? BM * sizeof(int64_t) : 0);
   static_assert(!REC || WM * WN * 64 >= BM, "a thread per tile row finds its cache position");
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
-  if (attr != hipSuccess) return attr;
+  static LdsLimit limit;
+  const hipError_t e = limit.raise(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>), int(kLds));
+  if (e != hipSuccess) return e;
   TileParams p{};
   p.a = g.a; p.lda = g.lda; p.w = REC ? g.w_f16p : g.w; p.scales = g.scales;
   p.m = m_end; p.n = g.n; p.k = g.k; p.epi = g.epi;
