@@ -642,6 +642,30 @@ def test_row_major_any_alignment(ops, m, n, k, int8):
         assert bool(((out.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m", [3, 17])
+def test_row_kernels_leave_grids_too_large_for_them(ops, m):
+    """2^29 + 1 columns: the row kernels' 64 columns per 512 threads would take 2^32
+    threads in one grid dimension; the skinny kernel takes the call."""
+    t = torch()
+    n, k = 2 ** 29 + 1, 8
+    say("too wide for the row kernels", m, n, k)
+    gen = t.Generator(device="cuda").manual_seed(m)
+    a = t.randn(m, k, generator=gen, device="cuda").half()
+    q = t.empty(k, n, dtype=t.int8, device="cuda").random_(-127, 128, generator=gen)
+    s = t.rand(n, generator=gen, device="cuda") * 1e-3
+    y = ops.gemm_int8(a, q, s)
+    good = []
+    for first in (0, n // 2 - 40, n - 200):
+        cut = slice(first, first + 200)
+        w = (q[:, cut].float() * s[cut]).half()
+        ref, size = a.double() @ w.double(), a.double().abs() @ w.double().abs()
+        bound = (k + 2) * 2.0 ** -24 * size
+        good.append(bool(((y[:, cut].double() - ref).abs() <= bound + 2.0 ** -11 * (ref.abs() + bound) + 2.0 ** -25).all()))
+    del q, s, y
+    t.cuda.empty_cache()
+    assert all(good)
+
+
 @pytest.mark.parametrize("kind,m,n,k,most", [
     ("fp16", 4, 3072, 2784, 6.9e-8), ("fp16", 4, 1600, 5648, 8.4e-8), ("fp16", 27, 5255, 3072, 8e-8),
     ("fp16", 31, 4800, 6400, 1.12e-7), ("int8", 12, 5170, 1600, 4.7e-8), ("int8", 27, 5255, 3072, 6.1e-8),

@@ -2329,9 +2329,11 @@ int skinny_splits(int m, int n, int k, size_t capacity) {
 // hundred weight rows), K split into equal whole-step ranges of at most
 // 4 x 16 steps; 8 waves when a split has at most 8 steps, else 16.  Depends
 // on N and K only.  hipErrorNotSupported when the shape does not fit (more
-// than kRowSplits splits, or partials beyond the pool): the caller then takes
-// the skinny kernel.
+// than kRowSplits splits, partials beyond the pool, or more threads than a grid
+// dimension holds): the caller then takes the skinny kernel.
 constexpr int kRowTargetBlocks = 192;
+// Threads of a launch in one dimension stay below this.
+constexpr int64_t kGridThreads = int64_t(1) << 32;
 template <bool INT8, bool WVEC, int W, int S>
 hipError_t launch_rowgemv_ws(const SkinnyParams& p, hipStream_t stream) {
   hipLaunchKernelGGL((rowgemv_kernel<INT8, WVEC, W, S>), dim3(unsigned(p.ntile) * unsigned(p.splits)), dim3(W * 64), 0, stream, p);
@@ -2352,6 +2354,7 @@ hipError_t launch_rowgemv(const GemmArgs& g, hipStream_t stream) {
   splits = (p.steps + spb - 1) / spb;
   if (splits > 1 && (p.ntile > kPoolTiles || int64_t(p.ntile) * splits * 1024 > int64_t(kPoolFloats)))
     return hipErrorNotSupported;
+  if (int64_t(p.ntile) * splits * (spb <= 8 ? 512 : 1024) >= kGridThreads) return hipErrorNotSupported;
   p.steps_per_block = spb;
   p.splits = splits;
   p.pool = splits > 1;
@@ -2396,7 +2399,7 @@ hipError_t launch_rowgemm(const GemmArgs& g, hipStream_t stream) {
   if (splits > 1 && units > kPoolTiles) splits = 1;
   const int spb = (p.steps + splits - 1) / splits;
   splits = (p.steps + spb - 1) / spb;
-  if (units * splits > INT_MAX / 2) return hipErrorNotSupported;
+  if (units * splits * (mt == 1 && spb > 8 ? 1024 : 512) >= kGridThreads) return hipErrorNotSupported;
   p.steps_per_block = spb;
   p.splits = splits;
   p.pool = splits > 1;
