@@ -2832,7 +2832,7 @@ struct F16GemmParams {
   int group_m;       // tile rows per group of the tile order
   int chunks_per_split, splits;
   bool defer;
-  bool pool;         // splits > 1 finish in this launch through the queue pool (EP == 1 only)
+  bool pool;         // splits > 1 finish in this launch through the queue pool
   Epilogue epi;
   float* partials;
 };
@@ -2855,14 +2855,15 @@ __global__ void pack_w16_kernel(const int8_t* q, int64_t ldq, const float* scale
   out[t] = __builtin_bit_cast(u32x4_t, v);
 }
 
-// Tile (WM * MT * 16) x (WN * R * 16), WM x WN waves, each MT x R MFMA blocks;
-// K in chunks of 32 moved HBM/L2 -> LDS by global_load_lds_dwordx4 (A
+// 64 x 64 tiles, 2 x 4 waves of 2 x 1 MFMA blocks each; K in chunks of 32 moved HBM/L2 -> LDS by global_load_lds_dwordx4 (A
 // fragments of 16 rows x 32 K in MFMA A order, B records as stored), S stages
 // as in the int8 panel kernel.  The epilogue runs from the accumulators.
-template <int WM, int WN, int MT, int R, int S, int EP = 1, int OCC = 2, bool POOL = false>
-__global__ __launch_bounds__(WM * WN * 64, OCC) void f16_gemm_kernel(F16GemmParams p) {
-  constexpr int W = WM * WN, NT = W * 64;
-  constexpr int BM = WM * MT * 16, BN = WN * R * 16;
+constexpr int kF16Waves = 8, kF16Tile = 64;
+template <int S, bool POOL = false>
+__global__ __launch_bounds__(kF16Waves * 64, 3) void f16_gemm_kernel(F16GemmParams p) {
+  constexpr int W = kF16Waves, WN = 4, MT = 2, R = 1, NT = W * 64;
+  constexpr int BM = kF16Tile, BN = kF16Tile;
+  static_assert(W / WN * MT * 16 == BM && WN * R * 16 == BN, "the waves' blocks make the tile");
   constexpr int NA = BM / 16, NB = BN / 16, NL = NA + NB;
   static_assert(NL % W == 0, "loads must split evenly over the waves");
   constexpr int LPW = NL / W;
@@ -2934,67 +2935,55 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void f16_gemm_kernel(F16GemmPara
   }
   wait_vmcnt<0>();
 
-  // Epilogue through an LDS fp32 tile of BM / EP rows x BN, EP passes (the
-  // accumulators never meet the epilogue's registers; EP > 1 cuts the LDS the
-  // kernel needs), each finished 4 columns per thread by tile_epilogue.
-  constexpr int PR = BM / EP;  // rows per pass
-  static_assert(BM % EP == 0 && PR % 16 == 0, "whole 16-row blocks per pass");
+  // Epilogue through an LDS fp32 tile (the accumulators never meet the
+  // epilogue's registers), finished 4 columns per thread by tile_epilogue.
   float* ctile = reinterpret_cast<float*>(lds);
+  __syncthreads();
 #pragma unroll
-  for (int pass = 0; pass < EP; ++pass) {
-    __syncthreads();
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int rb = (wm * MT + t) * 16 - pass * PR;  // block row inside this pass
-      if (rb < 0 || rb >= PR) continue;
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          ctile[(rb + 4 * g + v) * tile_pitch(BN) + (wn * R + r) * 16 + j] = acc[t][r][v];
+      for (int v = 0; v < 4; ++v)
+        ctile[((wm * MT + t) * 16 + 4 * g + v) * tile_pitch(BN) + (wn * R + r) * 16 + j] = acc[t][r][v];
+  __syncthreads();
+  if constexpr (POOL) {
+    if (p.splits > 1) {
+      if (tile_split_finish<BM, BN, NT>(ctile, split, p.splits, tm * p.tiles_n + tn))
+        tile_epilogue<BM, BN, NT>(p.epi, ctile, m0, cb0 * 16, p.m, p.n, bias, nullptr, split);
+      return;
     }
-    __syncthreads();
-    if constexpr (EP == 1 && POOL) {
-      if (p.splits > 1) {
-        if (tile_split_finish<PR, BN, NT>(ctile, split, p.splits, tm * p.tiles_n + tn))
-          tile_epilogue<PR, BN, NT>(p.epi, ctile, m0, cb0 * 16, p.m, p.n, bias, nullptr, split);
-        return;
-      }
-    }
-    tile_epilogue<PR, BN, NT>(p.epi, ctile, m0 + pass * PR, cb0 * 16, p.m, p.n, bias,
-                              epi_now ? nullptr : p.partials, split);
   }
+  tile_epilogue<BM, BN, NT>(p.epi, ctile, m0, cb0 * 16, p.m, p.n, bias, epi_now ? nullptr : p.partials, split);
 }
 
-template <int WM, int WN, int MT, int R, int S, int EP = 1, int OCC = 2>
+template <int S>
 hipError_t launch_f16_cfg(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* deferred) {
-  constexpr int BM = WM * MT * 16, BN = WN * R * 16;
+  constexpr int BM = kF16Tile, BN = kF16Tile;
   constexpr int NL = BM / 16 + BN / 16;
-  constexpr size_t kLds = std::max(size_t(S) * NL * 1024, size_t(BM / EP) * tile_pitch(BN) * 4);
+  constexpr size_t kLds = std::max(size_t(S) * NL * 1024, size_t(BM) * tile_pitch(BN) * 4);
   static LdsLimit limit, limit_pool;
-  hipError_t e = limit.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC>), int(kLds));
-  if (e == hipSuccess && EP == 1)
-    e = limit_pool.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC, EP == 1>), int(kLds));
+  hipError_t e = limit.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<S>), int(kLds));
+  if (e == hipSuccess) e = limit_pool.raise(reinterpret_cast<const void*>(&f16_gemm_kernel<S, true>), int(kLds));
   if (e != hipSuccess) return e;
   F16GemmParams p{};
   p.a = g.a; p.lda = g.lda; p.w = static_cast<const u32x4_t*>(g.w_f16p);
   p.m = g.m; p.n = g.n; p.k = g.k; p.epi = g.epi;
   p.kk = (g.k + 31) / 32;
   p.tiles_n = (g.n + BN - 1) / BN;
-  p.group_m = 2;  // M = 8192, 1600->6400: 315 us; row-major order 321, groups of 8 rows 327
+  p.group_m = 2;
   const int64_t tiles = int64_t(p.tiles_n) * ((g.m + BM - 1) / BM);
   if (tiles > (int64_t(1) << 28)) return hipErrorInvalidValue;
   p.tiles = int(tiles);
   int splits = 1;
   const bool pool = s && s->queue_pool && !deferred;
-  const size_t capacity = !pool ? ((s && s->partials) ? s->partial_floats : 0)
-                                : (EP == 1 && tiles <= kPoolTiles) ? kPoolFloats : 0;
+  const size_t capacity = !pool ? ((s && s->partials) ? s->partial_floats : 0) : tiles <= kPoolTiles ? kPoolFloats : 0;
   if (!g.canonical && capacity > 0 && tiles < 192) {
     splits = int(std::min<int64_t>((256 + tiles - 1) / tiles, std::max(1, p.kk / (S - 1))));
     while (splits > 1 && size_t(splits) * g.m * g.n > capacity) --splits;
     if (pool)
       splits = pool_splits(splits, tiles, BM * BN,
-                           kTileRounds * pool_max_splits(std::max(1, BM / (WM * WN * 64 / (BN / 4)))), p.kk);
+                           kTileRounds * pool_max_splits(std::max(1, BM / (kF16Waves * 64 / (BN / 4)))), p.kk);
   }
   p.chunks_per_split = (p.kk + splits - 1) / splits;
   splits = (p.kk + p.chunks_per_split - 1) / p.chunks_per_split;
@@ -3002,12 +2991,9 @@ hipError_t launch_f16_cfg(const GemmArgs& g, const Scratch* s, hipStream_t strea
   p.defer = deferred != nullptr && splits > 1;
   p.pool = pool;
   p.partials = s ? s->partials : nullptr;
-  if (pool && splits > 1)
-    hipLaunchKernelGGL((f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC, EP == 1>), dim3(unsigned(tiles * splits)),
-                       dim3(WM * WN * 64), kLds, stream, p);
-  else
-    hipLaunchKernelGGL((f16_gemm_kernel<WM, WN, MT, R, S, EP, OCC>), dim3(unsigned(tiles * splits)), dim3(WM * WN * 64),
-                       kLds, stream, p);
+  const dim3 grid(unsigned(tiles * splits)), block(kF16Waves * 64);
+  if (pool && splits > 1) hipLaunchKernelGGL((f16_gemm_kernel<S, true>), grid, block, kLds, stream, p);
+  else hipLaunchKernelGGL((f16_gemm_kernel<S>), grid, block, kLds, stream, p);
   if (p.defer) {
     *deferred = splits;
     return hipGetLastError();
@@ -3047,11 +3033,13 @@ struct TileParams {
 // chunk.  M = 8192, 1600->6400, int8: 207 us; groups of 2 / 4: 235 / 213.
 constexpr int kTileGroup = 8;
 
+// Rows of the records' epilogue passes.
+constexpr int kTilePassRows = 32;
 // LDS of a tile's operand rings, or of its epilogue's fp32 tile if larger.
-template <int TW, int BM, int BN, int EP>
+template <int TW, int BM, int BN>
 constexpr size_t tile_lds_ring() {
   constexpr size_t ring = size_t(2) * BM * 128 + size_t(TW == TW_REC16 ? 2 : 3) * BN * 128;
-  return TW == TW_REC16 ? std::max(ring, size_t(BM / EP) * tile_pitch(BN) * 4) : ring;
+  return TW == TW_REC16 ? std::max(ring, size_t(kTilePassRows) * tile_pitch(BN) * 4) : ring;
 }
 
 // Tile (WM * MT * 16) x (WN * R * 16), WM x WN waves of MT x R MFMA blocks,
@@ -3078,7 +3066,7 @@ constexpr size_t tile_lds_ring() {
 // M = 8192, 1600->6400: int8 row-major 517 -> 181 us (930 TF/s; the 64 x 64
 // kernel converted every weight once per 64 rows), fp16 row-major 511 -> 165 us,
 // fp16 records 228 -> 190 us; M = 2048, 768->3072, fp16 row-major 38 -> 19 us.
-template <int TW, int WM, int WN, int MT, int R, int EP, int OCC>
+template <int TW, int WM, int WN, int MT, int R, int OCC>
 __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams p) {
   constexpr int W = WM * WN, NT = W * 64;
   constexpr int BM = WM * MT * 16, BN = WN * R * 16, H = MT / 2;
@@ -3093,7 +3081,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
   // the cache position of each row of an EPI_QKV tile.
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   uint8_t* const blds = lds + 2 * ASTAGE;
-  int64_t* const kv_at = reinterpret_cast<int64_t*>(lds + tile_lds_ring<TW, BM, BN, EP>());
+  int64_t* const kv_at = reinterpret_cast<int64_t*>(lds + tile_lds_ring<TW, BM, BN>());
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
@@ -3321,7 +3309,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
   }
 
   if constexpr (REC) {
-    // Through an LDS fp32 tile of BM / EP rows x BN, EP passes.  A QKV tile's
+    // Through an LDS fp32 tile of kTilePassRows rows, BM / kTilePassRows passes.  A QKV tile's
     // cache positions (a search of row_start and three dependent loads each)
     // are found once per row here, not by every thread for each of its rows:
     // M = 2560, 1600->4800 80 -> 52 us.
@@ -3330,11 +3318,11 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
       kv_at[threadIdx.x] = m0 + int(threadIdx.x) < p.m ? qkv_row_position(p.epi, m0 + int(threadIdx.x)) : -1;
     float bias[4];
     load_bias4(p.epi, n0 + 4 * int(threadIdx.x % (BN / 4)), p.n, p.a, bias);
-    constexpr int PR = BM / EP;
-    static_assert(BM % EP == 0 && PR % 16 == 0, "whole 16-row blocks per pass");
+    constexpr int PR = kTilePassRows;
+    static_assert(BM % PR == 0 && PR % 16 == 0, "whole passes of whole 16-row blocks");
     float* ctile = reinterpret_cast<float*>(lds);
 #pragma unroll
-    for (int pass = 0; pass < EP; ++pass) {
+    for (int pass = 0; pass < BM / PR; ++pass) {
       __syncthreads();
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
@@ -3398,14 +3386,14 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void tile_gemm_kernel(TileParams
 }
 
 // Rows [m_begin, m_end) of the product.
-template <int TW, int WM, int WN, int MT, int R, int EP, int OCC>
+template <int TW, int WM, int WN, int MT, int R, int OCC>
 hipError_t launch_tile_cfg(const GemmArgs& g, int m_begin, int m_end, hipStream_t stream) {
   constexpr int BM = WM * MT * 16, BN = WN * R * 16;
   constexpr bool REC = TW == TW_REC16;
-  constexpr size_t kLds = tile_lds_ring<TW, BM, BN, EP>() + (REC ? BM * sizeof(int64_t) : 0);
+  constexpr size_t kLds = tile_lds_ring<TW, BM, BN>() + (REC ? BM * sizeof(int64_t) : 0);
   static_assert(!REC || WM * WN * 64 >= BM, "a thread per tile row finds its cache position");
   static LdsLimit limit;
-  const hipError_t e = limit.raise(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>), int(kLds));
+  const hipError_t e = limit.raise(reinterpret_cast<const void*>(&tile_gemm_kernel<TW, WM, WN, MT, R, OCC>), int(kLds));
   if (e != hipSuccess) return e;
   TileParams p{};
   p.a = g.a; p.lda = g.lda; p.w = REC ? g.w_f16p : g.w; p.scales = g.scales;
@@ -3416,7 +3404,7 @@ hipError_t launch_tile_cfg(const GemmArgs& g, int m_begin, int m_end, hipStream_
   const int64_t tiles = int64_t(p.tiles_n) * ((m_end - m_begin + BM - 1) / BM);
   if (tiles > (int64_t(1) << 28)) return hipErrorInvalidValue;
   p.tiles = int(tiles);
-  hipLaunchKernelGGL((tile_gemm_kernel<TW, WM, WN, MT, R, EP, OCC>), dim3(unsigned(tiles)), dim3(WM * WN * 64), kLds,
+  hipLaunchKernelGGL((tile_gemm_kernel<TW, WM, WN, MT, R, OCC>), dim3(unsigned(tiles)), dim3(WM * WN * 64), kLds,
                      stream, p);
   return hipGetLastError();
 }
@@ -3461,16 +3449,16 @@ template <int TW>
 hipError_t launch_tile(const GemmArgs& g, hipStream_t stream) {
   const int big = TW == TW_REC16 && g.k < 1024 ? 0 : tile_big_rows(g.m, g.n);
   if (big > 0) {
-    const hipError_t e = launch_tile_cfg<TW, 2, 4, 8, 4, 8, 2>(g, 0, std::min(big, g.m), stream);
+    const hipError_t e = launch_tile_cfg<TW, 2, 4, 8, 4, 2>(g, 0, std::min(big, g.m), stream);
     if (e != hipSuccess || big >= g.m) return e;
   }
   if constexpr (TW == TW_REC16) {
-    return launch_tile_cfg<TW, 2, 4, 4, 2, 4, 4>(g, big, g.m, stream);
+    return launch_tile_cfg<TW, 2, 4, 4, 2, 4>(g, big, g.m, stream);
   } else {
     const int64_t wide = tiles_of(g.m - big, g.n, 128, 256), cus = device_cus();
     if (TW == TW_ROW8 && 5 * wide >= 3 * cus && wide <= cus)
-      return launch_tile_cfg<TW, 2, 4, 4, 4, 4, 2>(g, big, g.m, stream);
-    return launch_tile_cfg<TW, 2, 2, 4, 4, 4, 2>(g, big, g.m, stream);
+      return launch_tile_cfg<TW, 2, 4, 4, 4, 2>(g, big, g.m, stream);
+    return launch_tile_cfg<TW, 2, 2, 4, 4, 2>(g, big, g.m, stream);
   }
 }
 
@@ -3591,8 +3579,8 @@ hipError_t launch_row_tiles(const GemmArgs& g, const Scratch* s, hipStream_t str
       !row_tiles_preferred<TW>(g, s))
     return hipErrorNotSupported;
   if (tiles_of(g.m, g.n, 128, 128) >= 144) return launch_tile<TW>(g, stream);
-  return TW == TW_ROW8 ? launch_tile_cfg<TW, 2, 2, 2, 4, 2, 2>(g, 0, g.m, stream)
-                       : launch_tile_cfg<TW, 2, 1, 2, 4, 2, 2>(g, 0, g.m, stream);
+  return TW == TW_ROW8 ? launch_tile_cfg<TW, 2, 2, 2, 4, 2>(g, 0, g.m, stream)
+                       : launch_tile_cfg<TW, 2, 1, 2, 4, 2>(g, 0, g.m, stream);
 }
 
 // Tile choice over the fp16 records, and when they beat the int8 panel
@@ -3614,8 +3602,8 @@ bool f16_gemm_preferred(int m, int n, int k) { return f16_gemm_large(m, n, k) ||
 
 hipError_t launch_f16(const GemmArgs& g, const Scratch* s, hipStream_t stream, int* deferred) {
   if (f16_gemm_large(g.m, g.n, g.k) && g.lda <= (1 << 22)) return launch_tile<TW_REC16>(g, stream);
-  if (g.k >= 1536) return launch_f16_cfg<2, 4, 2, 1, 4, 1, 3>(g, s, stream, deferred);
-  return launch_f16_cfg<2, 4, 2, 1, 3, 1, 3>(g, s, stream, deferred);
+  if (g.k >= 1536) return launch_f16_cfg<4>(g, s, stream, deferred);
+  return launch_f16_cfg<3>(g, s, stream, deferred);
 }
 
 template <bool INT8>
