@@ -388,10 +388,11 @@ def test_pack_w16_layout_bit_exact(ops, k, n):
                                    (8200, 256, 4000)])
 def test_f16_packed_prefill_gemm_against_oracle(ops, m, k, n):
     """Prefill GEMM over the pre-dequantised fp16 weights: ragged row and column
-    tiles, K a multiple of 32 but not of 64, the 256 x 256 tiles (K >= 4096,
-    192 of them) and the 256 x 128 tiles (1056 of them), bias / bias+GELU /
-    in-place residual epilogues against the oracle's int8 linear (the same
-    weight values)."""
+    tiles, K a multiple of 32 but not of 64, the 64 x 64 tiles (up to 512 rows and
+    short K), the 128-row tiles (1024 x 768 x 2304, 8200 x 256 x 4000) and whole
+    rounds of 256 x 256 ones before them (4100 x 1600 x 6400, 3000 x 4096 x 4000),
+    bias / bias+GELU / in-place residual epilogues against the oracle's int8 linear
+    (the same weight values)."""
     t = torch()
     rng = np.random.default_rng(13 * m + k + n)
     a = f16(rng.standard_normal((m, k)))
@@ -544,11 +545,14 @@ def test_layernorm_prologue_gemv_rejects_unsupported_shapes(ops):
     assert _ln_packed(*args(0, 64)) == 1
 
 
-# m, n, k of each tile choice of the large products, at ragged edges: 64-row tiles
-# (int8 over and up to 1024 rows, fp16), 128 x 128, 128 x 256 (int8), 256 x 256
-# in one round, and 256 x 256 tiles whose last round is 128-row tiles.
+# m, n, k at ragged edges.  First shapes of one to four chunks of K, where the
+# large tiles' pipeline only fills and drains (several of them now take the kernels
+# for few tiles or short K), then each tile choice over six and more chunks: 64-row
+# tiles, 128 x 128, 128 x 256 (int8), 256 x 256 in one round, and 256 x 256 tiles
+# whose last round is 128-row tiles.
 LARGE = [(1030, 260, 200), (1000, 1300, 136), (640, 644, 264), (1100, 2052, 72), (2047, 2560, 40),
-         (3601, 3844, 72), (5000, 3844, 40)]
+         (3601, 3844, 72), (5000, 3844, 40),
+         (1100, 1300, 456), (1500, 2052, 328), (2047, 2560, 328), (3601, 3844, 328), (5000, 3844, 392)]
 
 
 def large_reference(a, w, bias):
@@ -691,7 +695,11 @@ def test_few_rows_sum_in_short_chains(ops, kind, m, n, k, most):
     assert float((out.double() - ref).norm() / ref.norm()) <= most
 
 
-@pytest.mark.parametrize("m,n,k", [(1100, 2050, 96), (3601, 3841, 160), (5000, 3844, 32), (1100, 2050, 64)])
+@pytest.mark.parametrize("m,n,k", [
+    (1100, 2050, 96), (1100, 2050, 64),                         # 64 x 64 tiles
+    (3601, 3841, 160), (5000, 3844, 32), (1100, 2050, 352),     # 128-row tiles
+    (3601, 3841, 1056), (5000, 3844, 1120),                     # 256 x 256, alone and before 128-row tiles
+])
 def test_record_large_tiles(ops, m, n, k):
     """fp16 records: the value of every tile choice, and the bits of the
     row-major kernel where that takes the shape (one K order everywhere)."""
@@ -705,7 +713,7 @@ def test_record_large_tiles(ops, m, n, k):
     assert bool(((y.double() - ref).abs() <= bound + 2.0 ** -11 * (ref.abs() + bound) + 2.0 ** -25).all())
     if n % 4 == 0:
         assert t.equal(y, ops.gemm_int8(a, q, s, bias=bias))
-    few = 600  # 64 x 64 tiles, unsplit
+    few = 600  # other tiles, unsplit
     z = t.empty(few, n, dtype=t.float16, device="cuda")
     assert _w16(ops.lib, a[:few].contiguous(), packed, bias, z, None, few, n, k, 0) == 0
     assert t.equal(z, y[:few])
