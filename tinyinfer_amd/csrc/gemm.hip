@@ -12,15 +12,16 @@
 //    (standalone GEMV calls): no MFMA, 8 columns per workgroup, twice the
 //    workgroups of the 16-column MFMA blocks.
 //  * row GEMV / GEMM (M <= 1024, row-major weights of the C ABIs of either type
-//    and any alignment, 16-byte rows of A): about 192 workgroups, each one 64-column tile of 16 (M <= 64)
-//    or 32 rows over a range of 32-row K steps, every load of a wave's round
-//    in flight at once, the skinny kernel's fragments and MFMAs; K splits
-//    finish in the launch through the queue pool (rowgemv_kernel at M <= 16,
-//    rowgemm_kernel above).
+//    and any alignment, 16-byte rows of A): about 192 workgroups, each one
+//    64-column tile of 16 (M <= 64) or 32 rows over a range of 32-row K steps,
+//    every load of a wave's round in flight at once, the skinny kernel's
+//    fragments and MFMAs; K splits finish in the launch through the queue pool
+//    (rowgemv_kernel at M <= 16, rowgemm_kernel above, where row_gemm_preferred
+//    finds it faster than the tiled kernel).
 //  * skinny (M <= 32, row-major weights, where the row GEMV does not apply:
-//    unaligned operands, no queue pool): every wave streams weight fragments straight from
-//    HBM into MFMA B-operand registers (no LDS for weights), dequantises them in
-//    registers as fp16_rn(float(q) * scale[n]) and runs v_mfma_f32_16x16x32_f16
+//    unaligned operands, no queue pool, grids past the launch's limit): every wave
+//    streams weight fragments straight from HBM into MFMA B-operand registers (no
+//    LDS for weights), dequantises them in registers as fp16_rn(float(q) * scale[n]) and runs v_mfma_f32_16x16x32_f16
 //    with A padded to 16/32 rows.  A lane loads one dword (4 consecutive output
 //    columns) from 8 consecutive K rows, so the MFMA for "column slot" c covers
 //    columns {n0 + 4j + c}; the 4 waves of a workgroup split K, reduce through
@@ -32,11 +33,13 @@
 //    pool, written and read with agent-scope accesses, so no L2-wide
 //    writeback or invalidate is needed; queue_scratch.hpp).
 //  * large tiles (tile_gemm_kernel: row-major weights of either type and fp16
-//    records, where the grid of 64- to 256-row tiles fills the chip).
-//  * tiled (M > 32 where neither applies: unaligned operands, fp16 weights over
-//    few tiles): 64x64x32 tiles, A and the dequantised weight tile
-//    staged in LDS (weights transposed to [n][k] so both MFMA operands are one
-//    ds_read_b128 per lane), double buffered, same fused epilogues.
+//    records, where 64- to 256-row tiles are many enough: row_tiles_preferred,
+//    f16_gemm_large).
+//  * tiled (M > 32 where the others do not apply or are slower: unaligned operands,
+//    few columns whose K it splits, short K): 64x64x32 tiles, A and the
+//    dequantised weight tile staged in LDS (weights transposed to [n][k] so both
+//    MFMA operands are one ds_read_b128 per lane), double buffered, same fused
+//    epilogues.
 // Dequantisation mirrors reference kernels/src/cuda/tc/gemm.cu:21,24 and the
 // bias epilogue mirrors gemm.cu:73-80 / :118-124; accumulation is fp32.
 #include <algorithm>
@@ -563,7 +566,7 @@ __global__ __launch_bounds__(kSkinnyThreads) void skinny_kernel(SkinnyParams p) 
 // MFMA (the skinny kernel's fragments and dequantisation).  The waves meet in
 // LDS; with one split the workgroup runs the epilogue, otherwise each split's
 // sums go to the queue's pool slot and the tile's last split to arrive adds
-// them in split order (one round of loads) and runs it.  The plan depends on N
+// them by pairs (one round of loads) and runs it.  The plan depends on N
 // and K only, so a row's result does not depend on M.  fp16 weights (before, the
 // skinny kernel): M = 8 3072->768 9.0 -> 5.9 us; the tied head 768 x 50257, whose
 // rows start at any byte, at M = 4: 47 -> 18.5 us (int8).
@@ -646,8 +649,8 @@ __global__ __launch_bounds__(W * 64) void rowgemv_kernel(SkinnyParams p) {
 // steps w, w + W, ..., S of them per round with every load of the round in
 // flight before its first MFMA.  The waves meet in LDS; with one split the
 // workgroup runs the epilogue, otherwise each split's sums go to the queue's
-// pool slot as float4s and the unit's last split to arrive adds them in split
-// order (one round of loads) and runs it.  Row blocks are 16 rows up to M = 64,
+// pool slot as float4s and the unit's last split to arrive adds them by pairs
+// (one round of loads) and runs it.  Row blocks are 16 rows up to M = 64,
 // then 32; the K split follows the count of (tile, row block) units, so unlike
 // the M <= 16 GEMV a row's sums may differ between M values (the reference ABI
 // promises no batch invariance; the runtime never takes this path).  fp16 weights
@@ -3497,11 +3500,12 @@ int tiled_plan(const GemmArgs& g, const Scratch* s) {
 // split K over few tiles (us, this kernel against them):
 // * int8 up to kRowMaxM rows (the row GEMM): the tiles take about as long for 150
 //   of them (64 x 128) as for 512, K / 64 chunks of 1 us, the row GEMM what its
-//   M N K takes.  They meet at 140 + K / 12 tiles, at most 300, and at 300 where few
-//   rows share each weight from HBM: bias, 512 x 768 x 3072 (192 tiles) 17.9 /
-//   16.6, 768 x 768 x 3072 20 / 22, 866 x 3072 x 1600 53 / 35, 1000 x 1600 x 1600 30 /
-//   27, 523 x 2160 x 2304 41 / 25, 512 x 1600 x 4800 (304) 35 / 37, 590 x 4800 x 6400
-//   87 / 125, 208 x 584 x 6400 17.2 / 13.6, 283 x 928 x 6400 (250) 24.7 / 20;
+//   M N K takes.  They meet at 140 + K / 12 tiles, from K = 800 on later, at most
+//   300, and at 300 where few rows share each weight from HBM: bias, 512 x 768 x
+//   3072 (192 tiles) 17.9 / 16.6, 768 x 768 x 3072 20 / 22, 866 x 3072 x 1600 53 / 35,
+//   1000 x 1600 x 1600 30 / 27, 863 x 1328 x 2304 (252) 28 / 25, 523 x 2160 x 2304 41 /
+//   25, 512 x 1600 x 4800 (304) 35 / 37, 590 x 4800 x 6400 87 / 125, 208 x 584 x 6400
+//   17.2 / 13.6, 283 x 928 x 6400 (250) 24.7 / 20;
 // * fp16 up to kRowMaxM rows (the row GEMM, which loads twice the bytes): from
 //   160 such tiles, 1024 x 768 x 3072 18 / 24; the longest K keeps the row GEMM up
 //   to 144 tiles of 128 x 128;
@@ -3530,7 +3534,8 @@ bool row_tiles_preferred(const GemmArgs& g, const Scratch* s) {
     return false;
   if (g.m <= kRowMaxM) {
     const int64_t wide = tiles_of(g.m, g.n, 64, 128);
-    if (TW == TW_ROW8) return wide >= (g.m < 400 && g.k >= 400 ? 300 : std::min(140 + g.k / 12, 300));
+    const int64_t meet = std::min<int64_t>(std::max(140 + g.k / 12, 60 + g.k / 11 * 2), 300);
+    if (TW == TW_ROW8) return wide >= (g.m < 400 && g.k >= 400 ? 300 : meet);
     if (tiles_of(g.m, g.n, 128, 128) < 144 && (wide < 160 || g.k > 4096)) return false;
   }
   const int64_t tiles = tiles_of(g.m, g.n, 64, 64);

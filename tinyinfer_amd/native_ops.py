@@ -12,9 +12,10 @@ extent, device, integer argument or a tensor that requires grad,
 How it is built here: every native symbol is described by a string of
 parameter codes (``_ABI``); each call goes through a ``_Call`` that validates
 the operands in argument order, allocates outputs on the operands' device,
-records every tensor on the current torch stream (the caller's allocator must
-not recycle them while the queued kernels run), and appends that stream and the
-device index as the ABI's last two arguments.  There is no CPU path: the
+records the caller's tensors on the current torch stream (the allocator must not
+recycle them while the queued kernels run; outputs and metadata come from that
+stream's own pool), and appends that stream and the device index as the ABI's
+last two arguments.  There is no CPU path: the
 library must be built, and the operands must already live on the GPU.
 """
 from __future__ import annotations
